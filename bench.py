@@ -153,7 +153,8 @@ def workload(name, scheme="muscl"):
 
 
 def flux_pass_bytes(C, F, cfg):
-    """Algorithmic bytes of the first-stage launch of the fused flux/stage pass. Per cell: U (32)
+    """Algorithmic bytes of the first-stage launch of the flux/stage pass that reads gradients (order 3,
+    and the two-pass form of order 2). Per cell: U (32)
     + gradients (64) + area, 1/area (16) + face slots (8) read; new U (32) written, plus dt/area
     (8) with local time stepping and the accumulator (32) with RK4. Per face: L,R (8) + normal,
     length (24) + centre offset (16), plus the line stencil (16) for WENO5, whose faces read no
@@ -165,10 +166,26 @@ def flux_pass_bytes(C, F, cfg):
 
 
 def resid_pass_bytes(C, F, cfg):
-    """Algorithmic bytes of the flux pass in residual mode: per cell U (32) + gradients (64, MUSCL)
+    """Algorithmic bytes of that flux pass in residual mode: per cell U (32) + gradients (64, MUSCL)
     + area (8) + face slots (8) read, R (32) + local dt (8) written; per face L,R (8) + normal,
     length (24) + centre offset (16)."""
     return (32 + (64 if cfg["order"] == 2 else 0) + 8 + 8 + 32 + 8) * C + 48 * F
+
+
+def one_launch_bytes(C, F, cfg, resid):
+    """Algorithmic bytes of a second-order launch that forms its gradients itself. Per cell: U (32),
+    local neighbours and face slots (16) and the least-squares vectors (64), or the normals and
+    lengths (96), read; in residual mode area (8) read, R and dt (40) written; in the first stage
+    1/area (8) and, with local time stepping, area (8) read, new U (32), with local time stepping
+    dt/area (8) and with RK4 the accumulator (32) written; 1/area (8) for Green-Gauss where not read
+    already. Per face: local cells (4), normal, length and centre offset (40)."""
+    gg = cfg["gradient"] == "gg"
+    per_cell = 48 + (96 if gg else 64)
+    if resid:
+        per_cell += 48 + (8 if gg else 0)
+    else:
+        per_cell += 40 + (16 if cfg["lts"] else 0) + (32 if cfg["rk"] == 4 else 0)
+    return per_cell * C + 44 * F
 
 
 def apply_scheme(cfg, desc, scheme):
@@ -185,8 +202,8 @@ def apply_scheme(cfg, desc, scheme):
 
 
 def residual_contract(C, F, gradient, ms):
-    """One MUSCL residual evaluation (gradient pass + flux pass, each timed alone) against the
-    two-pass contract bytes B = 224 C + 80 F (Green-Gauss) or 224 C + 96 F (WLSQ), with C the
+    """One MUSCL residual evaluation (one launch, which forms its gradients) against the two-pass
+    contract bytes B = 224 C + 80 F (Green-Gauss) or 224 C + 96 F (WLSQ), with C the
     physical plus ghost cells and F all faces."""
     b = 224 * C + (96 if gradient == "wlsq" else 80) * F
     gbs = b / (ms / 1e3) / 1e9
@@ -412,7 +429,7 @@ def ffs_march_bench(args):
     rho = U[:, 0]
     p = 0.4 * (U[:, 3] - 0.5 * (U[:, 1] ** 2 + U[:, 2] ** 2) / rho)
     C, F = mesh.nphys, mesh.nfaces
-    step_bytes = 4 * (grad_pass_bytes(C, F, "gg") + flux_pass_bytes(C, F, cfg))
+    step_bytes = 4 * one_launch_bytes(C, F, cfg, False)
     out = {
         "metric": "step configuration march: cell-updates/s (2000 RK4 steps from the impulsive start)",
         "value": C * nsteps / wall, "unit": "cell-updates/s", "n_gpus": 1, "steps": nsteps, "warmup": 0,
@@ -422,7 +439,7 @@ def ffs_march_bench(args):
         "simulated_time": t_sim, "finite": bool(np.all(np.isfinite(U))),
         "min_density": float(rho.min()), "min_pressure": float(p.min()),
         "achieved_GBs": step_bytes / (wall / nsteps) / 1e9,
-        "achieved_note": "algorithmic bytes of 4 gradient + 4 fused flux/stage passes per step over the "
+        "achieved_note": "algorithmic bytes of 4 first-stage launches per step over the "
                          "wall time per step (host-timed, error norm read back every 250 steps)",
     }
     print(json.dumps(out), flush=True)
@@ -574,16 +591,16 @@ def fv_bench(args, wl, scheme, gradient, sub=False):
     torch.cuda.synchronize()
     err = s.step(1, history=True, stream=stream)[0][0]
     ok = bool(np.isfinite(err[0]))
-    contract = residual_contract(mesh.nphys + mesh.nghost, F, cfg["gradient"], ms_grad + ms_resid)
+    # at order 2 the residual-mode launch is the whole residual; WENO5's few gradients come before it
+    contract = residual_contract(mesh.nphys + mesh.nghost, F, cfg["gradient"],
+                                 ms_resid if cfg["order"] == 2 else ms_grad + ms_resid)
     contract_other = None
     if ffs and not sub:
         # the same residual with the other gradient (the step-mesh roofline run is defined for both)
         other = "gg" if cfg["gradient"] == "wlsq" else "wlsq"
         s.configure(mk(**dict(cfg, gradient=other)))
-        g2 = s.time_pass("grad", args.kernel_reps, stream=stream) / args.kernel_reps
         r2 = s.time_pass("resid", args.kernel_reps, stream=stream) / args.kernel_reps
-        contract_other = dict(residual_contract(mesh.nphys + mesh.nghost, F, other, g2 + r2), gradient=other,
-                              grad_ms=g2, resid_ms=r2)
+        contract_other = dict(residual_contract(mesh.nphys + mesh.nghost, F, other, r2), gradient=other, resid_ms=r2)
 
     t_step = ms_steps / 1e3 / args.steps
     launch_cfg = (f"workload={wl} tile={args.tile} face_budget={args.face_budget} "
@@ -592,9 +609,10 @@ def fv_bench(args, wl, scheme, gradient, sub=False):
                   + (f" scheme={scheme}" if scheme != "muscl" else "") + (" positivity=1" if pos else ""))
     value = F * nres / t_step
     # with the fallback the stage pass is its detecting pass, which also writes one flag byte per cell
-    bflux = flux_pass_bytes(C, F, cfg) + (C if pos else 0)
+    one = cfg["order"] == 2
+    bflux = (one_launch_bytes(C, F, cfg, False) if one else flux_pass_bytes(C, F, cfg)) + (C if pos else 0)
     achieved = bflux / (ms_flux / 1e3) / 1e9
-    bres = resid_pass_bytes(C, F, cfg)
+    bres = one_launch_bytes(C, F, cfg, True) if one else resid_pass_bytes(C, F, cfg)
     out = {
         "metric": "time to residual 1e-8: NN-warm vs plain (batched); FP64 face-flux evals/s",
         "value": value,
@@ -623,9 +641,10 @@ def fv_bench(args, wl, scheme, gradient, sub=False):
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": measured_traffic((wl, scheme), launch_cfg),
-                     "kernel": ("flux_tile_kernel, the positivity fallback's detecting pass (fused face flux + "
+                     "kernel": ("flux_tile_kernel (face flux + gather + RK stage), first stage" if scheme == "weno" else
+                                "fused_tile_kernel, the positivity fallback's detecting pass (gradients + face flux + "
                                 "gather + RK stage + admissibility flags), first stage" if pos else
-                                "flux_tile_kernel (fused face flux + gather + RK stage), first stage"),
+                                "fused_tile_kernel (gradients + face flux + gather + RK stage), first stage"),
                      "algorithmic_bytes_per_launch": bflux, "avg_launch_ms": ms_flux,
                      "traffic_source": PROFILES.get((wl, scheme))},
         "grad_pass": {"avg_launch_ms": ms_grad,

@@ -162,12 +162,21 @@ int cfd_mesh_create(int npts, const double *pts3, int ncells, const int *cells4,
     *out = nullptr;
     const Layout &L = m->lay;
     hipError_t e = hipSuccess;
-    std::vector<double> geo, w;
+    std::vector<double> geo, cw, fd;
     std::vector<int> lr;
-    pack_face_records(L, 0, geo, w, lr);
+    pack_face_geometry(L, 0, geo, lr);
+    cell_face_vectors(L, cw);
+    face_offsets(L, fd);
+    TileRings rings;
+    tile_rings(m->ref, L, rings);
     if ((e = upload(&m->d_tile_cstart, L.tile_cstart)) != hipSuccess ||
         (e = upload(&m->d_tile_fstart, L.tile_fstart)) != hipSuccess ||
-        (e = upload(&m->d_fgeo, geo)) != hipSuccess || (e = upload(&m->d_fw, w)) != hipSuccess ||
+        (e = upload(&m->d_fgeo, geo)) != hipSuccess || (e = upload(&m->d_cw, cw)) != hipSuccess ||
+        (e = upload(&m->d_fd, fd)) != hipSuccess ||
+        (e = upload(&m->d_rings, rings.tiles)) != hipSuccess || (e = upload(&m->d_ring_cell, rings.cell)) != hipSuccess ||
+        (e = upload(&m->d_own_nbr, rings.own)) != hipSuccess || (e = upload(&m->d_ring_nbr, rings.ring)) != hipSuccess ||
+        (e = upload(&m->d_ghost, rings.ghost)) != hipSuccess ||
+        (e = upload(&m->d_ghost_n, rings.ghost_n)) != hipSuccess || (e = upload(&m->d_floc, rings.face)) != hipSuccess ||
         (e = upload(&m->d_fLR, lr)) != hipSuccess || (e = upload(&m->d_fnx, L.fnx)) != hipSuccess ||
         (e = upload(&m->d_fny, L.fny)) != hipSuccess || (e = upload(&m->d_fdl, L.fdl)) != hipSuccess ||
         (e = upload(&m->d_slots, L.slots)) != hipSuccess ||
@@ -201,7 +210,19 @@ int cfd_mesh_create(int npts, const double *pts3, int ncells, const int *cells4,
     d.tile_cstart = m->d_tile_cstart;
     d.tile_fstart = m->d_tile_fstart;
     d.fgeo = reinterpret_cast<const double2 *>(m->d_fgeo);
-    d.fw = reinterpret_cast<const double2 *>(m->d_fw);
+    d.cw = reinterpret_cast<const double2 *>(m->d_cw);
+    if (rings.ok) {
+        d.rings = reinterpret_cast<const int4 *>(m->d_rings);
+        d.ring_cell = m->d_ring_cell;
+        d.own_nbr = reinterpret_cast<const ushort4 *>(m->d_own_nbr);
+        d.ring_nbr = reinterpret_cast<const ushort4 *>(m->d_ring_nbr);
+        d.ghost = reinterpret_cast<const int2 *>(m->d_ghost);
+        d.ghost_n = reinterpret_cast<const double2 *>(m->d_ghost_n);
+        d.fd = reinterpret_cast<const double2 *>(m->d_fd);
+        d.floc = reinterpret_cast<const ushort2 *>(m->d_floc);
+        d.max_local = rings.max_local;
+        d.max_grad = rings.max_grad;
+    }
     d.fLR = reinterpret_cast<const int2 *>(m->d_fLR);
     d.fnx = m->d_fnx;
     d.fny = m->d_fny;
@@ -336,13 +357,22 @@ static int ensure_line_stencils(cfd_mesh_s *m) {
     return 0;
 }
 
-// Gradient pass of a time step: at order 3 only over the tiles whose gradients a MUSCL face
+// Face normals and lengths per cell on the device (first Green-Gauss configuration at order 2).
+static int ensure_cell_normals(cfd_mesh_s *m) {
+    std::lock_guard<std::mutex> lock(m->lazy);
+    if (m->d_cn || !m->dev.rings) return 0;
+    std::vector<double> cn;
+    cell_face_normals(m->lay, cn);
+    HIP_TRY(upload(&m->d_cn, cn));
+    m->dev.cn = m->d_cn;
+    return 0;
+}
+
+// Gradient pass of a time step at order 3: only over the tiles whose gradients a MUSCL face
 // reads (none on an all-quadrilateral line mesh away from its boundary).
 static int step_grad(cfd_solver_s *s, const double4 *in, hipStream_t st) {
     const cfd_config_t &c = s->cfg;
-    if (c.order == 2) {
-        HIP_TRY(launch_grad(s->dev, s->dcfg, c.gradient, in, s->grad, c.block, st));
-    } else if (c.order == 3 && c.viscous) {  // every face reads gradients
+    if (c.order == 3 && c.viscous) {  // every face reads gradients
         HIP_TRY(launch_grad(s->dev, s->dcfg, c.gradient, in, s->grad, c.block, st));
     } else if (c.order == 3 && s->ngtiles > 0) {
         DevMesh dm = s->dev;
@@ -359,6 +389,7 @@ int cfd_solver_configure(cfd_solver_t *s, const cfd_config_t *cfg) {
     int rc = check_config(s->m, cfg);
     if (rc) return rc;
     if (cfg->order == 3 && (rc = ensure_line_stencils(s->m))) return rc;
+    if (cfg->order == 2 && cfg->gradient == GRAD_GG && (rc = ensure_cell_normals(s->m))) return rc;
     {
         std::lock_guard<std::mutex> lock(s->m->lazy);
         s->dev = s->m->dev;
@@ -508,13 +539,18 @@ static int dt_pass_order(const cfd_config_t &c) { return c.viscous ? 2 : 1; }
 
 // residual of state `in` into s->R, s->dt (+ minimum dt into *dtmin when set)
 static int residual_pass(cfd_solver_s *s, const double4 *in, double *dtmin, const double4 *uexit,
-                         hipStream_t st, int order_override = 0) {
+                         hipStream_t st, int order_override = 0, bool want_grad = false) {
     const cfd_config_t &c = s->cfg;
     const int order = order_override ? order_override : c.order;
     if (c.ref_mode && order == 2 && c.flux == FLUX_ROE) return ref_roe2o_pass(s, in, dtmin, uexit, st);
-    if (order >= 2) HIP_TRY(launch_grad(s->dev, s->dcfg, c.gradient, in, s->grad, c.block, st));
     StageArgs a = resid_args(s, dtmin != nullptr, uexit);
-    HIP_TRY(launch_flux(s->dev, s->dcfg, c.flux, order, c.limiter, MODE_RESID, in, s->grad, a, c.block, st));
+    if (order == 2) {
+        HIP_TRY(launch_second_order(s->dev, s->dcfg, c.flux, c.limiter, c.gradient, MODE_RESID, in, s->grad, want_grad,
+                                    a, 0, c.block, st));
+    } else {
+        if (order == 3) HIP_TRY(launch_grad(s->dev, s->dcfg, c.gradient, in, s->grad, c.block, st));
+        HIP_TRY(launch_flux(s->dev, s->dcfg, c.flux, order, c.limiter, MODE_RESID, in, s->grad, a, c.block, st));
+    }
     if (dtmin) HIP_TRY(launch_min_reduce(s->dt_partial, s->dev.ntiles, dtmin, st));
     return 0;
 }
@@ -523,7 +559,7 @@ int cfd_residual(cfd_solver_t *s, double *R, double *dt, double *grad, void *str
     if (!s) return fail(CFD_E_ARG, "cfd_residual: null solver");
     if (!s->has_state) return fail(CFD_E_STATE, "cfd_residual: state not set");
     hipStream_t st = (hipStream_t)stream;
-    int rc = residual_pass(s, s->Un, nullptr, nullptr, st);
+    int rc = residual_pass(s, s->Un, nullptr, nullptr, st, 0, grad != nullptr);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(st));
     const int nc = s->m->ref.nc;
@@ -645,7 +681,8 @@ static int native_step(cfd_solver_s *s, bool want_err, hipStream_t st) {
     for (int k = 0; k < nst; k++) {
         const double4 *in = (nst == 4) ? ins4[k] : ins3[k];
         double4 *out = (nst == 4) ? outs4[k] : outs3[k];
-        if (int rc = step_grad(s, in, st)) return rc;
+        if (c.order == 3)
+            if (int rc = step_grad(s, in, st)) return rc;
         StageArgs a{};
         a.rk = nst;
         a.stage = k;
@@ -666,9 +703,13 @@ static int native_step(cfd_solver_s *s, bool want_err, hipStream_t st) {
             a.pflag = s->pflag;
             a.dirty = s->dirty;
             a.pos_range = pos_flags(s);
-            HIP_TRY(launch_flux_pos(dm, s->dcfg, c.flux, c.limiter, 1, in, s->grad, a, c.block, st));
-            HIP_TRY(launch_flux_pos(dm, s->dcfg, c.flux, c.limiter, 2, in, s->grad, a, c.block, st));
+            for (int pass = 1; pass <= 2; pass++)
+                HIP_TRY(launch_second_order(dm, s->dcfg, c.flux, c.limiter, c.gradient, MODE_STAGE, in, s->grad, false, a,
+                                            pass, c.block, st));
             s->pos_seq++;
+        } else if (c.order == 2) {
+            HIP_TRY(launch_second_order(dm, s->dcfg, c.flux, c.limiter, c.gradient, MODE_STAGE, in, s->grad, false, a, 0,
+                                        c.block, st));
         } else {
             HIP_TRY(launch_flux(dm, s->dcfg, c.flux, c.order, c.limiter, MODE_STAGE, in, s->grad, a, c.block, st));
         }
@@ -741,7 +782,16 @@ int cfd_time_pass(cfd_solver_t *s, int which, int reps, float *ms, void *stream)
         if (rc) return rc;
         s->dt_valid = true;
     }
+    // the two-pass form's stage and residual launches are timed without their gradient pass
+    const bool one_launch = c.order == 2 && fused_fits(dm, s->dcfg, c.gradient, c.block);
     if (c.order >= 2) HIP_TRY(launch_grad(dm, s->dcfg, c.gradient, s->Un, s->grad, c.block, st));
+    auto stage = [&](int mode, const StageArgs &sa, int pos) {
+        if (one_launch)
+            return launch_second_order(dm, s->dcfg, c.flux, c.limiter, c.gradient, mode, s->Un, s->grad, false, sa, pos,
+                                       c.block, st);
+        if (pos) return launch_flux_pos(dm, s->dcfg, c.flux, c.limiter, pos, s->Un, s->grad, sa, c.block, st);
+        return launch_flux(dm, s->dcfg, c.flux, c.order, c.limiter, mode, s->Un, s->grad, sa, c.block, st);
+    };
     StageArgs a{};
     a.rk = (c.rk == 4) ? 4 : 3;
     a.stage = 0;
@@ -768,12 +818,8 @@ int cfd_time_pass(cfd_solver_t *s, int which, int reps, float *ms, void *stream)
     HIP_TRY(hipEventRecord(e0, st));
     for (int r = 0; r < reps; r++) {
         if (which == 0) HIP_TRY(launch_grad(dm, s->dcfg, c.gradient, s->Un, s->grad, c.block, st));
-        else if (which == 1 && pos) HIP_TRY(launch_flux_pos(dm, s->dcfg, c.flux, c.limiter, 1, s->Un, s->grad, a, c.block, st));
-        else if (which == 1) HIP_TRY(launch_flux(dm, s->dcfg, c.flux, c.order, c.limiter, MODE_STAGE, s->Un, s->grad, a, c.block, st));
-        else if (which == 3) {
-            const StageArgs r = resid_args(s, false, nullptr);
-            HIP_TRY(launch_flux(dm, s->dcfg, c.flux, c.order, c.limiter, MODE_RESID, s->Un, s->grad, r, c.block, st));
-        }
+        else if (which == 1) HIP_TRY(stage(MODE_STAGE, a, pos ? 1 : 0));
+        else if (which == 3) HIP_TRY(stage(MODE_RESID, resid_args(s, false, nullptr), 0));
         else {
             int rc = native_step(s, false, st);
             if (rc) return rc;
@@ -782,7 +828,7 @@ int cfd_time_pass(cfd_solver_t *s, int which, int reps, float *ms, void *stream)
     }
     HIP_TRY(hipEventRecord(e1, st));
     if (which == 1 && pos) {
-        HIP_TRY(launch_flux_pos(dm, s->dcfg, c.flux, c.limiter, 2, s->Un, s->grad, a, c.block, st));
+        HIP_TRY(stage(MODE_STAGE, a, 2));
         s->pos_seq++;
     }
     HIP_TRY(hipEventSynchronize(e1));

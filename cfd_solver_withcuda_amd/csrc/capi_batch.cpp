@@ -74,11 +74,14 @@ struct cfd_batch_s {
     std::vector<int> iperm;      // caller cell (global) -> renumbered cell (global)
     // device mesh
     int *d_tile_cstart = nullptr, *d_tile_fstart = nullptr;
-    double *d_fgeo = nullptr, *d_fw = nullptr, *d_area = nullptr, *d_inv_area = nullptr;
+    double *d_fgeo = nullptr, *d_cw = nullptr, *d_cn = nullptr, *d_ghost_n = nullptr, *d_fd = nullptr, *d_area = nullptr, *d_inv_area = nullptr;
     double *d_fnx = nullptr, *d_fny = nullptr, *d_fdl = nullptr;
     int *d_fLR = nullptr;
     int *d_fst = nullptr;  // WENO line stencils, 4 per face entry (order 3)
     uint16_t *d_slots = nullptr;
+    // tile neighbourhoods (TileRings), order 2
+    int *d_rings = nullptr, *d_ring_cell = nullptr, *d_ghost = nullptr;
+    uint16_t *d_own_nbr = nullptr, *d_ring_nbr = nullptr, *d_floc = nullptr;
     int *d_tile_inst = nullptr, *d_inst_tile = nullptr, *d_tile_list = nullptr, *d_tile_count = nullptr;
     int *d_inst_off = nullptr, *d_status = nullptr, *d_steps = nullptr;
     int *d_fz = nullptr, *d_fz_since = nullptr;  // per instance limiter-freezing state
@@ -112,7 +115,7 @@ struct cfd_batch_s {
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
         if (stream) (void)hipStreamDestroy(stream);
-        void *ps[] = {d_tile_cstart, d_tile_fstart, d_fgeo, d_fw, d_fnx, d_fny, d_fdl, d_fLR, d_fst, d_area, d_inv_area, d_slots, d_tile_inst, d_inst_tile,
+        void *ps[] = {d_tile_cstart, d_tile_fstart, d_fgeo, d_cw, d_cn, d_ghost_n, d_fd, d_rings, d_ring_cell, d_ghost, d_own_nbr, d_ring_nbr, d_floc, d_fnx, d_fny, d_fdl, d_fLR, d_fst, d_area, d_inv_area, d_slots, d_tile_inst, d_inst_tile,
                       d_tile_list, d_tile_count, d_inst_off, d_status, d_steps, d_inst_fs, d_err4,
                       Un, Ua, Ub, acc, grad, hbuf, err_partial, d_fz, d_fz_since, d_fz_best, psi,
                       Uc, acc2, pflag, dirty};
@@ -162,7 +165,15 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
     const int ni = (int)in.size();
     std::vector<Layout> lays(ni);
     std::vector<std::vector<int>> sts(ni);  // WENO line stencils (order 3)
+    std::vector<TileRings> rgs(ni);         // tile neighbourhoods (order 2)
+    struct Packed {                         // the instance's device records
+        std::vector<double> geo, cw, cn, fd;
+        std::vector<int> lr;
+    };
+    std::vector<Packed> pks(ni);
     std::vector<std::string> errs(ni);
+    std::vector<long> first_cell(ni + 1, 0);
+    for (int i = 0; i < ni; i++) first_cell[i + 1] = first_cell[i] + in[i].ncells;
     {
         std::atomic<int> next{0};
         auto work = [&]() {
@@ -174,6 +185,14 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
                     build_ref_mesh(in[i].npts, in[i].pts, in[i].ncells, in[i].cells, rm);
                     build_layout(rm, tile, 1, lays[i], face_budget);
                     if (cfg.order == 3) line_stencils(rm, lays[i], sts[i]);
+                    Packed &pk = pks[i];
+                    pack_face_geometry(lays[i], (int)first_cell[i], pk.geo, pk.lr);
+                    if (cfg.order >= 2) cell_face_vectors(lays[i], pk.cw);
+                    if (cfg.order == 2) {
+                        tile_rings(rm, lays[i], rgs[i]);
+                        face_offsets(lays[i], pk.fd);
+                        if (cfg.gradient == GRAD_GG) cell_face_normals(lays[i], pk.cn);
+                    }
                 } catch (const std::exception &e) {
                     errs[i] = e.what();
                 }
@@ -203,6 +222,17 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
         fe_off[i + 1] = fe_off[i] + (int)lays[i].fL.size();
         b->max_tile_faces = std::max(b->max_tile_faces, lays[i].max_tile_faces);
     }
+    // offsets of the instances' ring cells and ghosts
+    bool rings = cfg.order == 2;
+    std::vector<size_t> rc_off(ni + 1, 0), gh_off(ni + 1, 0);
+    for (int i = 0; i < ni; i++) {
+        rings = rings && rgs[i].ok;
+        rc_off[i + 1] = rc_off[i] + rgs[i].cell.size();
+        gh_off[i + 1] = gh_off[i] + rgs[i].ghost.size() / 2;
+        b->dev.max_local = std::max(b->dev.max_local, rgs[i].max_local);
+        b->dev.max_grad = std::max(b->dev.max_grad, rgs[i].max_grad);
+    }
+    rings = rings && rc_off[ni] <= 0x7FFFFFFFu;
     b->nc = b->cell_off[ni];
     b->ntiles = b->inst_tile[ni];
     b->nfe = fe_off[ni];
@@ -216,7 +246,18 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
     BALLOC(b->d_tile_cstart, nt + 1);
     BALLOC(b->d_tile_fstart, nt + 1);
     BALLOC(b->d_fgeo, 6 * nfe);
-    BALLOC(b->d_fw, 4 * nfe);
+    if (cfg.order >= 2) BALLOC(b->d_cw, 8 * nc);
+    if (rings) {
+        BALLOC(b->d_rings, 4 * nt);
+        BALLOC(b->d_ring_cell, rc_off[ni]);
+        BALLOC(b->d_own_nbr, 4 * nc);
+        BALLOC(b->d_ring_nbr, 4 * rc_off[ni]);
+        BALLOC(b->d_ghost, 2 * gh_off[ni]);
+        BALLOC(b->d_ghost_n, 2 * gh_off[ni]);
+        BALLOC(b->d_floc, 2 * nfe);
+        BALLOC(b->d_fd, 2 * nfe);
+        if (cfg.gradient == GRAD_GG) BALLOC(b->d_cn, 12 * nc);
+    }
     BALLOC(b->d_fLR, 2 * nfe);
     BALLOC(b->d_fnx, nfe);
     BALLOC(b->d_fny, nfe);
@@ -268,9 +309,29 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
             tc[t] = L.tile_cstart[t] + cb;
             tf[t] = L.tile_fstart[t] + fb;
         }
-        std::vector<double> geo, w;
-        std::vector<int> lr;
-        pack_face_records(L, cb, geo, w, lr);
+        Packed &pk = pks[i];
+        if (rings) {
+            TileRings &rg = rgs[i];
+            for (size_t t = 0; t < nti; t++) {
+                rg.tiles[4 * t] += (int)rc_off[i];
+                rg.tiles[4 * t + 3] += (int)gh_off[i];
+            }
+            for (int &v : rg.cell) v += cb;
+            for (size_t g = 0; g < rg.ghost.size(); g += 2) rg.ghost[g] += cb;
+            if ((e = h2d(b->d_rings + 4 * (size_t)tb, rg.tiles.data(), rg.tiles.size())) != hipSuccess ||
+                (e = h2d(b->d_ring_cell + rc_off[i], rg.cell.data(), rg.cell.size())) != hipSuccess ||
+                (e = h2d(b->d_own_nbr + 4 * (size_t)cb, rg.own.data(), rg.own.size())) != hipSuccess ||
+                (e = h2d(b->d_ring_nbr + 4 * rc_off[i], rg.ring.data(), rg.ring.size())) != hipSuccess ||
+                (e = h2d(b->d_ghost + 2 * gh_off[i], rg.ghost.data(), rg.ghost.size())) != hipSuccess ||
+                (e = h2d(b->d_ghost_n + 2 * gh_off[i], rg.ghost_n.data(), rg.ghost_n.size())) != hipSuccess ||
+                (e = h2d(b->d_floc + 2 * (size_t)fb, rg.face.data(), rg.face.size())) != hipSuccess ||
+                (e = h2d(b->d_fd + 2 * (size_t)fb, pk.fd.data(), pk.fd.size())) != hipSuccess ||
+                (b->d_cn && (e = h2d(b->d_cn + 12 * (size_t)cb, pk.cn.data(), pk.cn.size())) != hipSuccess)) {
+                delete b;
+                return capi_hip_fail(e, "cfd_batch_create upload");
+            }
+            rg = TileRings();
+        }
         if (cfg.order == 3) {
             std::vector<int> &st = sts[i];
             for (int &v : st)
@@ -285,9 +346,9 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
         if ((e = h2d(b->d_tile_cstart + tb, tc.data(), nti)) != hipSuccess ||
             (e = h2d(b->d_tile_fstart + tb, tf.data(), nti)) != hipSuccess ||
             (e = h2d(b->d_tile_inst + tb, ti.data(), nti)) != hipSuccess ||
-            (e = h2d(b->d_fgeo + 6 * (size_t)fb, geo.data(), 6 * nfi)) != hipSuccess ||
-            (e = h2d(b->d_fw + 4 * (size_t)fb, w.data(), 4 * nfi)) != hipSuccess ||
-            (e = h2d(b->d_fLR + 2 * (size_t)fb, lr.data(), 2 * nfi)) != hipSuccess ||
+            (e = h2d(b->d_fgeo + 6 * (size_t)fb, pk.geo.data(), 6 * nfi)) != hipSuccess ||
+            (b->d_cw && (e = h2d(b->d_cw + 8 * (size_t)cb, pk.cw.data(), pk.cw.size())) != hipSuccess) ||
+            (e = h2d(b->d_fLR + 2 * (size_t)fb, pk.lr.data(), 2 * nfi)) != hipSuccess ||
             (e = h2d(b->d_fnx + fb, L.fnx.data(), nfi)) != hipSuccess ||
             (e = h2d(b->d_fny + fb, L.fny.data(), nfi)) != hipSuccess ||
             (e = h2d(b->d_fdl + fb, L.fdl.data(), nfi)) != hipSuccess ||
@@ -297,7 +358,8 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
             delete b;
             return capi_hip_fail(e, "cfd_batch_create upload");
         }
-        L = Layout();  // release this instance's host copy
+        L = Layout();  // release this instance's host copies
+        pk = Packed();
     }
     const int last_c = b->nc, last_f = b->nfe;
     std::vector<double4> fsv(ni);
@@ -319,7 +381,18 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
     d.tile_cstart = b->d_tile_cstart;
     d.tile_fstart = b->d_tile_fstart;
     d.fgeo = reinterpret_cast<const double2 *>(b->d_fgeo);
-    d.fw = reinterpret_cast<const double2 *>(b->d_fw);
+    d.cw = reinterpret_cast<const double2 *>(b->d_cw);
+    if (rings) {
+        d.rings = reinterpret_cast<const int4 *>(b->d_rings);
+        d.ring_cell = b->d_ring_cell;
+        d.own_nbr = reinterpret_cast<const ushort4 *>(b->d_own_nbr);
+        d.ring_nbr = reinterpret_cast<const ushort4 *>(b->d_ring_nbr);
+        d.ghost = reinterpret_cast<const int2 *>(b->d_ghost);
+        d.ghost_n = reinterpret_cast<const double2 *>(b->d_ghost_n);
+        d.fd = reinterpret_cast<const double2 *>(b->d_fd);
+        d.floc = reinterpret_cast<const ushort2 *>(b->d_floc);
+        d.cn = b->d_cn;
+    }
     d.fLR = reinterpret_cast<const int2 *>(b->d_fLR);
     d.fst = reinterpret_cast<const int4 *>(b->d_fst);
     d.fnx = b->d_fnx;
@@ -388,7 +461,7 @@ int batch_step_launches(cfd_batch_s *b, double tol, int grid_tiles) {
     for (int k = 0; k < nst; k++) {
         const double4 *in = (nst == 4) ? ins4[k] : ins3[k];
         double4 *out = (nst == 4) ? outs4[k] : outs3[k];
-        if (c.order >= 2) BHIP(launch_grad(dm, dc, c.gradient, in, b->grad, b->block, b->stream));
+        if (c.order == 3) BHIP(launch_grad(dm, dc, c.gradient, in, b->grad, b->block, b->stream));
         StageArgs a{};
         a.rk = nst;
         a.stage = k;
@@ -407,8 +480,12 @@ int batch_step_launches(cfd_batch_s *b, double tol, int grid_tiles) {
             a.pflag = b->pflag;
             a.dirty = b->dirty;
             a.pos_range = (c.positivity == 1 ? 1 : 0) | (k << 1) | (((k + 1) % nst) << 3);
-            BHIP(launch_flux_pos(dm, dc, c.flux, c.limiter, 1, in, b->grad, a, b->block, b->stream));
-            BHIP(launch_flux_pos(dm, dc, c.flux, c.limiter, 2, in, b->grad, a, b->block, b->stream));
+            for (int pass = 1; pass <= 2; pass++)
+                BHIP(launch_second_order(dm, dc, c.flux, c.limiter, c.gradient, MODE_STAGE, in, b->grad, false, a, pass,
+                                         b->block, b->stream));
+        } else if (c.order == 2) {
+            BHIP(launch_second_order(dm, dc, c.flux, c.limiter, c.gradient, MODE_STAGE, in, b->grad, false, a, 0, b->block,
+                                     b->stream));
         } else {
             BHIP(launch_flux(dm, dc, c.flux, c.order, c.limiter, MODE_STAGE, in, b->grad, a, b->block, b->stream));
         }

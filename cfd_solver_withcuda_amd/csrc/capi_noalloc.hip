@@ -75,14 +75,14 @@ extern "C" int cfd_residual_noalloc(const cfd_mesh_t *m, const cfd_config_t *cfg
     hipStream_t st = (hipStream_t)stream;
     const double4 *U = static_cast<const double4 *>(d_U);
     hipError_t e;
-    if (cfg->order >= 2 && (e = launch_grad(dm, dc, cfg->gradient, U, grad, cfg->block, st)) != hipSuccess)
-        return capi_hip_fail(e, "cfd_residual_noalloc: gradient pass");
     StageArgs a{};
     a.R_out = static_cast<double *>(d_R);
     a.dt_out = static_cast<double *>(d_dt);
     a.dt_partial = d_dtmin ? dt_partial : nullptr;
-    if ((e = launch_flux(dm, dc, cfg->flux, cfg->order, cfg->limiter, MODE_RESID, U, grad, a, cfg->block, st)) != hipSuccess)
-        return capi_hip_fail(e, "cfd_residual_noalloc: flux pass");
+    e = cfg->order == 2 ? launch_second_order(dm, dc, cfg->flux, cfg->limiter, cfg->gradient, MODE_RESID, U, grad, false,
+                                              a, 0, cfg->block, st)
+                        : launch_flux(dm, dc, cfg->flux, 1, cfg->limiter, MODE_RESID, U, grad, a, cfg->block, st);
+    if (e != hipSuccess) return capi_hip_fail(e, "cfd_residual_noalloc: residual pass");
     if (d_dtmin && (e = launch_min_reduce(dt_partial, dm.ntiles, static_cast<double *>(d_dtmin), st)) != hipSuccess)
         return capi_hip_fail(e, "cfd_residual_noalloc: time-step minimum");
     return 0;

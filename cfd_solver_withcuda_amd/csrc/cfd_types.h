@@ -44,12 +44,24 @@ struct DevMesh {
     // The gradient pass reads only what it needs, from compact arrays:
     const int2 *fLR;          // [nfe] {L, R}
     const double *fnx, *fny, *fdl;  // [nfe] unit normal and length (Green-Gauss, WLSQ ghosts)
-    const double2 *fw;        // [2*nfe] least-squares coefficient vectors of L (2e) and R (2e+1)
+    const double2 *cw;        // [4*nc] least-squares coefficient vector of each cell's faces, slot order
     // WENO (order 3) only: per face entry the line stencil {L-1, L-2, R+1, R+2} (renumbered
     // cells through opposite faces of quadrilaterals), all -1 where the line is incomplete
     const int4 *fst;          // [nfe]
     const uint16_t *slots;    // [4*nc] (local face << 1) | (cell is R); 0xFFFF = none
     const double *area, *inv_area;  // [nc]
+    // Tile neighbourhoods (mesh_host.h, TileRings), for the passes that form a tile's gradients
+    // themselves; rings is null where a tile has too many local cells
+    const int4 *rings;        // [ntiles] {ring start, n1 | ghosts << 16, nr, ghost start}
+    const int *ring_cell;     // ring cells (first ring, then second) of the tiles in turn
+    const ushort4 *own_nbr;   // [nc] local neighbours of each cell, face order; 0xFFFF = none
+    const ushort4 *ring_nbr;  // [ring cells] the same of the first-ring cells
+    const int2 *ghost;        // {owner cell, face kind} of the tiles' ghosts
+    const double2 *ghost_n;   // their outward unit normals
+    const double2 *fd;        // [nfe] centre offset x_R - x_L (ghost: reflected centre)
+    const ushort2 *floc;      // [nfe] local cells of L and R (R: the ghost on a boundary face)
+    const double *cn;         // [12*nc] outward unit normal and length per face slot (Green-Gauss; lazily built)
+    int max_local, max_grad;  // most local cells, and cells with gradients, of a tile
     // Batched meshes (several independent instances concatenated; null for one mesh):
     const int *tile_inst;     // [ntiles] instance of each tile
     const double4 *inst_fs;   // [ninst] prescribed state (rho, u, v, p) of each instance

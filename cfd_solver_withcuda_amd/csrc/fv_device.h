@@ -46,6 +46,12 @@ __device__ __forceinline__ void state_from_U(double U0, double U1, double U2, do
     s.U[3] = U3;
 }
 
+// Sound speed of a cell state, with state_from_U's arithmetic.
+__device__ __forceinline__ double sound_speed(double rho, double p) {
+    const double inv = 1.0 / rho;
+    return sqrt(kGamma * p * inv);
+}
+
 // Density and pressure of a conserved state, with state_from_U's arithmetic.
 __device__ __forceinline__ void rho_p_of(const double *U, double &rho, double &p) {
     double Rho = U[0];
@@ -458,7 +464,8 @@ __device__ __forceinline__ double limited_slope(double a, double b) {
 // slope; freeze = 1 records psi[k] = slope / c (0 where c = 0), rounded to FP32; freeze = 2 uses
 // slope = psi[k] * c (smooth in the state, so steady marches do not stall on limiter switching).
 // FP32 factors halve the frozen march's extra reads.
-template <int LIM>
+// CELL_SOUND: c holds its sound speed (otherwise the fallback forms it).
+template <int LIM, bool CELL_SOUND = true>
 __device__ __forceinline__ void reconstruct_side(const FState &c, const FState &o, const double *g,
                                                  double dx, double dy, double sgn, int freeze,
                                                  float *psi, FState &out) {
@@ -479,7 +486,9 @@ __device__ __forceinline__ void reconstruct_side(const FState &c, const FState &
     }
     if (!(Wf[0] > 0.0) || !(Wf[3] > 0.0)) {
         // first order on this side: the cell's primitives, conserved values formed from them
-        for (int k = 0; k < 5; k++) out.W[k] = c.W[k];
+        for (int k = 0; k < 4; k++) out.W[k] = c.W[k];
+        if constexpr (CELL_SOUND) out.W[4] = c.W[4];
+        else out.W[4] = sound_speed(c.W[0], c.W[3]);
         cons_from_prim(c.W[0], c.W[1], c.W[2], c.W[3], out.U);
         return;
     }

@@ -94,11 +94,12 @@ __device__ __forceinline__ void load_state(const double4 *__restrict__ U, int c,
     state_from_U(u.x, u.y, u.z, u.w, s);
 }
 
-// Block-wide sum of 4 values per thread into out[0..3] (fixed tree order). `red` holds
-// 4 * blockDim.x doubles of LDS.
-__device__ __forceinline__ void block_sum4(double *red, const double *v, double *out) {
-    const int t = threadIdx.x, n = blockDim.x;
-    for (int k = 0; k < 4; k++) red[k * n + t] = v[k];
+// Sum of 4 values of each of a workgroup's first n threads (n a power of two) into out[0..3] (fixed
+// tree order). `red` holds 4 n doubles of LDS.
+__device__ __forceinline__ void block_sum4(double *red, const double *v, double *out, int n) {
+    const int t = threadIdx.x;
+    if (t < n)
+        for (int k = 0; k < 4; k++) red[k * n + t] = v[k];
     __syncthreads();
     for (int s = n / 2; s > 0; s >>= 1) {
         if (t < s)
@@ -109,9 +110,9 @@ __device__ __forceinline__ void block_sum4(double *red, const double *v, double 
         for (int k = 0; k < 4; k++) out[k] = red[k * n];
 }
 
-__device__ __forceinline__ double block_min(double *red, double v) {
-    const int t = threadIdx.x, n = blockDim.x;
-    red[t] = v;
+__device__ __forceinline__ double block_min(double *red, double v, int n) {
+    const int t = threadIdx.x;
+    if (t < n) red[t] = v;
     __syncthreads();
     for (int s = n / 2; s > 0; s >>= 1) {
         if (t < s) red[t] = fmin(red[t], red[t + s]);
@@ -374,6 +375,59 @@ __device__ __forceinline__ void flux_face(const DevMesh &m, const DevCfg &cfg,
     for (int q = 0; q < 4; q++) sF[q * FT + j] = F[q];
 }
 
+// One Runge-Kutta stage of cell c: Uo from the step's start Un, the stage input us (TVD-RK3's later
+// stages), the net flux r and h = dt / area; RK4 keeps its weighted sum of net fluxes in st.acc_*
+// (a4: the sum so far, of its later stages).
+__device__ __forceinline__ void stage_update(const StageArgs &st, int c, double h, const double *Un, const double *us,
+                                             const double4 &a4, const double *r, double *Uo) {
+    if (st.rk == 4) {
+        double acc[4] = {a4.x, a4.y, a4.z, a4.w};
+        for (int q = 0; q < 4; q++) {
+            switch (st.stage) {
+            case 0: acc[q] = r[q]; Uo[q] = Un[q] - 0.5 * h * r[q]; break;
+            case 1: acc[q] += 2.0 * r[q]; Uo[q] = Un[q] - 0.5 * h * r[q]; break;
+            case 2: acc[q] += 2.0 * r[q]; Uo[q] = Un[q] - h * r[q]; break;
+            default: Uo[q] = Un[q] - (h / 6.0) * (acc[q] + r[q]); break;
+            }
+        }
+        if (st.stage < 3) st.acc_out[c] = make_double4(acc[0], acc[1], acc[2], acc[3]);
+    } else {
+        for (int q = 0; q < 4; q++) {
+            switch (st.stage) {
+            case 0: Uo[q] = Un[q] - h * r[q]; break;
+            case 1: Uo[q] = 0.75 * Un[q] + 0.25 * (us[q] - h * r[q]); break;
+            default: Uo[q] = (1.0 / 3.0) * Un[q] + (2.0 / 3.0) * (us[q] - h * r[q]); break;
+            }
+        }
+    }
+}
+
+// Positivity fallback: a stage state is inadmissible without a positive density and pressure, or
+// (range) outside the relaxed range of the neighbourhood's densities and pressures.
+__device__ __forceinline__ bool inadmissible(const double *Uo, double rlo, double rhi, double plo, double phi,
+                                             bool range) {
+    double rn, pn;
+    rho_p_of(Uo, rn, pn);
+    const double dr = fmax(1e-3 * fabs(rhi), 1e-3 * (rhi - rlo));
+    const double dp = fmax(1e-3 * fabs(phi), 1e-3 * (phi - plo));
+    return !(rn > 0.0) || !(pn > 0.0) ||
+           (range && (!(rn >= rlo - dr && rn <= rhi + dr) || !(pn >= plo - dp && pn <= phi + dp)));
+}
+
+// Marks the tile of an inadmissible cell and the tiles of its face neighbours (slots sls): they
+// recompute the stage.
+__device__ __forceinline__ void mark_dirty(const DevMesh &m, const StageArgs &st, int tile, int c0, int nct, int fs,
+                                           const uint16_t *sls) {
+    st.dirty[tile] = 1;
+    for (int f = 0; f < 4; f++) {
+        const uint16_t sl = sls[f];
+        if (sl == 0xFFFF) break;
+        const int4 a = reinterpret_cast<const int4 *>(m.fgeo)[3 * (size_t)(fs + (sl >> 1))];
+        const int o = (sl & 1) ? a.x : a.y;
+        if (o >= 0 && (unsigned)(o - c0) >= (unsigned)nct) st.dirty[tile_of_cell(m, o)] = 1;
+    }
+}
+
 // FZ: the stage reads st.freeze and can record or use frozen limiter factors (launched only when a
 // freezing state is set; without it the kernel holds none of that code). Exit ghosts from
 // st.Uexit (the reference iteration's stages) exist in residual mode only.
@@ -540,35 +594,14 @@ __global__ void __launch_bounds__(256) CFD_FLUX_ATTR CFD_POS_ATTR flux_tile_kern
                 h = (*st.dt_global) * ia;
             }
             const double Un[4] = {un4.x, un4.y, un4.z, un4.w};
+            const double us[4] = {u4.x, u4.y, u4.z, u4.w};
             double Uo[4];
-            if (st.rk == 4) {
-                double4 a4 = (st.stage == 0) ? make_double4(0, 0, 0, 0) : st.acc_in[c];
-                double acc[4] = {a4.x, a4.y, a4.z, a4.w};
-                for (int q = 0; q < 4; q++) {
-                    switch (st.stage) {
-                    case 0: acc[q] = r[q]; Uo[q] = Un[q] - 0.5 * h * r[q]; break;
-                    case 1: acc[q] += 2.0 * r[q]; Uo[q] = Un[q] - 0.5 * h * r[q]; break;
-                    case 2: acc[q] += 2.0 * r[q]; Uo[q] = Un[q] - h * r[q]; break;
-                    default: Uo[q] = Un[q] - (h / 6.0) * (acc[q] + r[q]); break;
-                    }
-                }
-                if (st.stage < 3) st.acc_out[c] = make_double4(acc[0], acc[1], acc[2], acc[3]);
-            } else {
-                const double us[4] = {u4.x, u4.y, u4.z, u4.w};
-                for (int q = 0; q < 4; q++) {
-                    switch (st.stage) {
-                    case 0: Uo[q] = Un[q] - h * r[q]; break;
-                    case 1: Uo[q] = 0.75 * Un[q] + 0.25 * (us[q] - h * r[q]); break;
-                    default: Uo[q] = (1.0 / 3.0) * Un[q] + (2.0 / 3.0) * (us[q] - h * r[q]); break;
-                    }
-                }
-            }
+            const double4 a4 = (st.rk == 4 && st.stage > 0) ? st.acc_in[c] : make_double4(0, 0, 0, 0);
+            stage_update(st, c, h, Un, us, a4, r, Uo);
             if constexpr (POS == 1) {
                 // positivity fallback, detection: the stage state must have a positive density and
                 // pressure within the relaxed range of the cell's and its face neighbours' stage
                 // inputs (the same test as the oracle's stage_fallback_flags)
-                double rn, pn;
-                rho_p_of(Uo, rn, pn);
                 const float *nb = reinterpret_cast<const float *>(sNb);
                 double rlo = (double)(float)sW[k], rhi = rlo, plo = (double)(float)sW[3 * T + k], phi = plo;
                 for (int f = 0; f < 4; f++) {
@@ -583,23 +616,9 @@ __global__ void __launch_bounds__(256) CFD_FLUX_ATTR CFD_POS_ATTR flux_tile_kern
                     plo = fmin(plo, pj);
                     phi = fmax(phi, pj);
                 }
-                const double dr = fmax(1e-3 * fabs(rhi), 1e-3 * (rhi - rlo));
-                const double dp = fmax(1e-3 * fabs(phi), 1e-3 * (phi - plo));
-                const bool bad = !(rn > 0.0) || !(pn > 0.0) ||
-                                 ((st.pos_range & 1) && (!(rn >= rlo - dr && rn <= rhi + dr) ||
-                                                         !(pn >= plo - dp && pn <= phi + dp)));
+                const bool bad = inadmissible(Uo, rlo, rhi, plo, phi, st.pos_range & 1);
                 st.pflag[c] = bad ? 1 : 0;
-                if (bad) {
-                    // this tile and the tiles of the cell's face neighbours recompute the stage
-                    st.dirty[tile] = 1;
-                    for (int f = 0; f < 4; f++) {
-                        const uint16_t sl = sls[f];
-                        if (sl == 0xFFFF) break;
-                        const int4 a = reinterpret_cast<const int4 *>(m.fgeo)[3 * (size_t)(fs + (sl >> 1))];
-                        const int o = (sl & 1) ? a.x : a.y;
-                        if (o >= 0 && (unsigned)(o - c0) >= (unsigned)nct) st.dirty[tile_of_cell(m, o)] = 1;
-                    }
-                }
+                if (bad) mark_dirty(m, st, tile, c0, nct, fs, sls);
             }
             st.Uout[c] = make_double4(Uo[0], Uo[1], Uo[2], Uo[3]);
             if (st.last) {
@@ -629,21 +648,21 @@ __global__ void __launch_bounds__(256) CFD_FLUX_ATTR CFD_POS_ATTR flux_tile_kern
     if constexpr (MODE == MODE_RESID) {
         if (st.dt_partial) {
             __syncthreads();
-            double b = block_min(smem, dtmin);
+            double b = block_min(smem, dtmin, B);
             if (threadIdx.x == 0) st.dt_partial[tile] = b;
         }
     } else {
         if (st.last && st.err_partial) {
             __syncthreads();
             double out[4];
-            block_sum4(smem, errp, out);
+            block_sum4(smem, errp, out, B);
             if (threadIdx.x == 0)
                 for (int q = 0; q < 4; q++) st.err_partial[4 * tile + q] = out[q];
             __syncthreads();
         }
         if (st.last && st.dt_partial) {
             __syncthreads();
-            double b = block_min(smem, dtmin);
+            double b = block_min(smem, dtmin, B);
             if (threadIdx.x == 0) st.dt_partial[tile] = b;
         }
     }

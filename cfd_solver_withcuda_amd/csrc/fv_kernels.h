@@ -52,6 +52,14 @@ size_t flux_launch_smem(const DevMesh &m, int order, int grad_lds, int block, bo
 hipError_t launch_flux_pos(const DevMesh &m, const DevCfg &c, int flux, int lim, int pass,
                            const double4 *Us, const double *grad, const StageArgs &st, int block,
                            hipStream_t s);
+// Second-order passes: the residual (R, dt and, when grad_out, the gradients) or one stage with
+// pos = 0, or the positivity fallback's pass pos = 1 or 2. Where the tiles' neighbourhoods fit
+// (fused_fits) a pass is one launch (fv_fused.h); otherwise a gradient pass into `grad` comes first
+// (not before pos = 2, which reads pass 1's).
+bool fused_fits(const DevMesh &m, const DevCfg &c, int gradient, int block);
+hipError_t launch_second_order(const DevMesh &m, const DevCfg &c, int flux, int lim, int gradient, int mode,
+                               const double4 *Us, double *grad, bool grad_out, const StageArgs &st, int pos,
+                               int block, hipStream_t s);
 hipError_t launch_grad(const DevMesh &m, const DevCfg &c, int grad_type, const double4 *Us,
                        double *grad, int block, hipStream_t s);
 hipError_t launch_flux(const DevMesh &m, const DevCfg &c, int flux, int order, int lim, int mode,

@@ -14,7 +14,7 @@
 
 #include <algorithm>
 
-#include "fv_flux.h"
+#include "fv_fused.h"
 
 namespace cfd {
 
@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(256) grad_tile_kernel(DevMesh m, DevCfg cfg,
             for (int f = 0; f < 4; f++) {
                 const uint16_t sl = sls[f];
                 if (sl == 0xFFFF) break;
-                const double2 w = m.fw[2 * (size_t)(fs + (sl >> 1)) + (sl & 1)];
+                const double2 w = m.cw[4 * (size_t)c + f];
                 ga[f] = w.x;
                 gb[f] = w.y;
             }
@@ -349,7 +349,7 @@ __global__ void __launch_bounds__(256) roe2o_kernel(int nc, const RefCells rc, c
         dt[c] = dtc;
     }
     if (dt_partial) {
-        const double b = block_min(red, dtc);
+        const double b = block_min(red, dtc, blockDim.x);
         if (threadIdx.x == 0) dt_partial[blockIdx.x] = b;
     }
 }
@@ -554,7 +554,7 @@ __global__ void __launch_bounds__(256) ref_update_kernel(int nc, int kind, int l
     }
     if (kind >= 2) {
         double out[4];
-        block_sum4(red, e, out);
+        block_sum4(red, e, out, blockDim.x);
         if (threadIdx.x == 0)
             for (int q = 0; q < 4; q++) err_partial[4 * blockIdx.x + q] = out[q];
     }
@@ -630,6 +630,44 @@ hipError_t launch_flux(const DevMesh &m, const DevCfg &c, int flux, int order, i
     if (order == 2 && c.viscous) return launch_flux_visc(m, c, flux, lim, mode, Us, grad, st, block, sm, s);
     if (order == 1) return launch_flux_family<1, false>(m, c, flux, lim, mode, Us, grad, st, block, sm, s);
     return launch_flux_family<2, false>(m, c, flux, lim, mode, Us, grad, st, block, sm, s);
+}
+
+// The one-launch pass runs where its LDS lets at least two workgroups share a compute unit, and
+// not with persistent workgroups (a launch mode of the two-pass kernels).
+bool fused_fits(const DevMesh &m, const DevCfg &c, int gradient, int block) {
+    if (!m.rings || c.persist || (gradient == GRAD_GG && !m.cn)) return false;
+    return sizeof(double) * fused_doubles(m.max_local, m.max_grad, m.max_tile_faces, block, block) <= 65536;
+}
+
+// Threads of a one-launch pass: the configuration's block, except where the launch leaves compute
+// units idle (no more tiles than compute units; the recomputing pass, of few tiles): there the time
+// is one tile's chain of arithmetic, and one thread per face shortens it.
+static int fused_threads(const DevMesh &m, const DevCfg &c, int block, int most, bool few) {
+    constexpr int kComputeUnits = 256;
+    if (!few && grid_of(m, c) > kComputeUnits) return block;
+    return std::max(block, std::min(most, (m.max_tile_faces + 63) / 64 * 64));
+}
+
+hipError_t launch_second_order(const DevMesh &m, const DevCfg &c, int flux, int lim, int gradient, int mode,
+                               const double4 *Us, double *grad, bool grad_out, const StageArgs &st, int pos,
+                               int block, hipStream_t s) {
+    // exit ghosts from another state (the reference iteration's stages): only the two-pass form
+    // takes different ghosts for gradients and fluxes
+    if (!fused_fits(m, c, gradient, block) || (mode == MODE_RESID && st.Uexit)) {
+        if (pos != 2) {
+            const hipError_t e = launch_grad(m, c, gradient, Us, grad, block, s);
+            if (e != hipSuccess) return e;
+        }
+        return pos ? launch_flux_pos(m, c, flux, lim, pos, Us, grad, st, block, s)
+                   : launch_flux(m, c, flux, 2, lim, mode, Us, grad, st, block, s);
+    }
+    FusedArgs a{m, c, Us, grad_out ? grad : nullptr, st, gradient == GRAD_GG, block};
+    const int threads = fused_threads(m, c, block, c.viscous || pos == 2 ? 512 : 1024, pos == 2);
+    const size_t sm = sizeof(double) * fused_doubles(m.max_local, m.max_grad, m.max_tile_faces, threads, block);
+    if (pos) return launch_fused_pos(a, flux, lim, pos, threads, sm, s);
+    if (mode == MODE_STAGE && st.freeze) return launch_fused_freeze(a, flux, lim, c.viscous != 0, threads, sm, s);
+    return c.viscous ? launch_fused_visc(a, flux, lim, mode, threads, sm, s)
+                     : launch_fused_plain(a, flux, lim, mode, threads, sm, s);
 }
 
 hipError_t launch_fill(double *p, double v, int n, hipStream_t s) {

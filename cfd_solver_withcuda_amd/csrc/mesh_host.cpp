@@ -415,6 +415,118 @@ void build_layout(const RefMesh &m, int tile, int renumber, Layout &L, int face_
     L.tile_fstart[L.ntiles] = (int)L.fL.size();
 }
 
+void tile_rings(const RefMesh &m, const Layout &L, TileRings &r) {
+    r = TileRings();
+    const int nc = m.nc;
+    r.tiles.reserve(4 * (size_t)L.ntiles);
+    r.cell.reserve(nc);
+    r.own.assign(4 * (size_t)nc, 0xFFFF);
+    r.face.assign(2 * L.fL.size(), 0xFFFF);
+    std::vector<int> mark(nc, -1), lid(nc, 0);
+    // renumbered neighbour of renumbered cell k across its face f, or -1 at a boundary
+    auto across = [&](int k, int f) {
+        const int j = m.nbr[4 * (size_t)L.perm[k] + f];
+        return j < nc ? L.iperm[j] : -1;
+    };
+    auto faces = [&](int k) { return m.nf[L.perm[k]]; };
+    for (int t = 0; t < L.ntiles; t++) {
+        const int k0 = L.tile_cstart[t], k1 = L.tile_cstart[t + 1], nct = k1 - k0;
+        const size_t r0 = r.cell.size(), g0 = r.ghost.size() / 2;
+        for (int k = k0; k < k1; k++) {
+            mark[k] = t;
+            lid[k] = k - k0;
+        }
+        auto add_ring = [&](int k) {
+            for (int f = 0; f < faces(k); f++) {
+                const int j = across(k, f);
+                if (j < 0 || mark[j] == t) continue;
+                mark[j] = t;
+                lid[j] = nct + (int)(r.cell.size() - r0);
+                r.cell.push_back(j);
+            }
+        };
+        for (int k = k0; k < k1; k++) add_ring(k);
+        const int n1 = (int)(r.cell.size() - r0);
+        for (int i = 0; i < n1; i++) add_ring(r.cell[r0 + i]);
+        const int nr = (int)(r.cell.size() - r0);
+        r.ring.resize(4 * r.cell.size(), 0xFFFF);
+        int ng = 0;
+        for (int i = 0; i < nct + n1; i++) {
+            const int k = i < nct ? k0 + i : r.cell[r0 + i - nct];
+            const int c = L.perm[k];
+            uint16_t *out = i < nct ? &r.own[4 * (size_t)k] : &r.ring[4 * (r0 + i - nct)];
+            for (int f = 0; f < m.nf[c]; f++) {
+                const int j = across(k, f);
+                if (j >= 0) {
+                    out[f] = (uint16_t)lid[j];
+                    continue;
+                }
+                out[f] = (uint16_t)(nct + nr + ng++);
+                r.ghost.push_back(k);
+                r.ghost.push_back(m.kind[4 * (size_t)c + f]);
+                r.ghost_n.push_back(m.nrm[8 * (size_t)c + 2 * f]);
+                r.ghost_n.push_back(m.nrm[8 * (size_t)c + 2 * f + 1]);
+            }
+        }
+        if (nct + nr + ng >= 0xFFFF || n1 > 0xFFFF || ng > 0x7FFF || r.cell.size() > 0x7FFFFFFFu) {
+            r = TileRings();
+            return;
+        }
+        for (int e = L.tile_fstart[t]; e < L.tile_fstart[t + 1]; e++) {
+            r.face[2 * (size_t)e] = (uint16_t)lid[L.fL[e]];
+            if (L.fR[e] >= 0) r.face[2 * (size_t)e + 1] = (uint16_t)lid[L.fR[e]];
+        }
+        for (int k = k0; k < k1; k++)
+            for (int f = 0; f < faces(k); f++) {
+                const int e = L.tile_fstart[t] + (L.slots[4 * (size_t)k + f] >> 1);
+                if (L.fR[e] < 0) r.face[2 * (size_t)e + 1] = r.own[4 * (size_t)k + f];
+            }
+        const int rec[4] = {(int)r0, n1 | (ng << 16), nr, (int)g0};
+        r.tiles.insert(r.tiles.end(), rec, rec + 4);
+        r.max_local = std::max(r.max_local, nct + nr + ng);
+        r.max_grad = std::max(r.max_grad, nct + n1);
+    }
+    r.ok = true;
+}
+
+// Calls f(cell, slot, face entry, cell is the entry's right cell) for every used face slot.
+template <typename F>
+static void each_slot(const Layout &L, F f) {
+    for (int t = 0; t < L.ntiles; t++)
+        for (int k = L.tile_cstart[t]; k < L.tile_cstart[t + 1]; k++)
+            for (int s = 0; s < 4; s++) {
+                const uint16_t sl = L.slots[4 * (size_t)k + s];
+                if (sl == 0xFFFF) break;
+                f((size_t)k, s, (size_t)L.tile_fstart[t] + (sl >> 1), (bool)(sl & 1));
+            }
+}
+
+void cell_face_vectors(const Layout &L, std::vector<double> &w) {
+    w.assign(8 * L.area.size(), 0.0);
+    each_slot(L, [&](size_t k, int s, size_t e, bool right) {
+        const double *v = right ? &L.fwR[2 * e] : &L.fwL[2 * e];
+        w[8 * k + 2 * s] = v[0];
+        w[8 * k + 2 * s + 1] = v[1];
+    });
+}
+
+void cell_face_normals(const Layout &L, std::vector<double> &n) {
+    n.assign(12 * L.area.size(), 0.0);
+    each_slot(L, [&](size_t k, int s, size_t e, bool right) {
+        n[12 * k + 3 * s] = right ? -L.fnx[e] : L.fnx[e];
+        n[12 * k + 3 * s + 1] = right ? -L.fny[e] : L.fny[e];
+        n[12 * k + 3 * s + 2] = L.fdl[e];
+    });
+}
+
+void face_offsets(const Layout &L, std::vector<double> &d) {
+    d.resize(2 * L.fdx.size());
+    for (size_t e = 0; e < L.fdx.size(); e++) {
+        d[2 * e] = L.fdx[e];
+        d[2 * e + 1] = L.fdy[e];
+    }
+}
+
 // The physical cell across the face opposite slot f of quadrilateral c, or -1.
 static int cell_behind(const RefMesh &m, int c, int f) {
     if (c < 0 || f < 0 || m.nf[c] != 4) return -1;
@@ -448,11 +560,9 @@ void line_stencils(const RefMesh &m, const Layout &L, std::vector<int> &st) {
     }
 }
 
-void pack_face_records(const Layout &L, int cell_off, std::vector<double> &geo, std::vector<double> &w,
-                       std::vector<int> &lr) {
+void pack_face_geometry(const Layout &L, int cell_off, std::vector<double> &geo, std::vector<int> &lr) {
     const size_t n = L.fL.size();
     geo.resize(6 * n);
-    w.resize(4 * n);
     lr.resize(2 * n);
     for (size_t e = 0; e < n; e++) {
         lr[2 * e] = L.fL[e] + cell_off;
@@ -463,6 +573,15 @@ void pack_face_records(const Layout &L, int cell_off, std::vector<double> &geo, 
         geo[6 * e + 3] = L.fdl[e];
         geo[6 * e + 4] = L.fdx[e];
         geo[6 * e + 5] = L.fdy[e];
+    }
+}
+
+void pack_face_records(const Layout &L, int cell_off, std::vector<double> &geo, std::vector<double> &w,
+                       std::vector<int> &lr) {
+    pack_face_geometry(L, cell_off, geo, lr);
+    const size_t n = L.fL.size();
+    w.resize(4 * n);
+    for (size_t e = 0; e < n; e++) {
         w[4 * e] = L.fwL[2 * e];
         w[4 * e + 1] = L.fwL[2 * e + 1];
         w[4 * e + 2] = L.fwR[2 * e];

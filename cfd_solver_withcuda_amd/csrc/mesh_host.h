@@ -51,6 +51,34 @@ void build_layout(const RefMesh &m, int tile, int renumber, Layout &L, int face_
 // dx, dy), w gets 4 (the least-squares vectors of L, then of R), lr gets {L, R}.
 void pack_face_records(const Layout &L, int cell_off, std::vector<double> &geo, std::vector<double> &w,
                        std::vector<int> &lr);
+// geo and lr alone.
+void pack_face_geometry(const Layout &L, int cell_off, std::vector<double> &geo, std::vector<int> &lr);
+
+// Neighbourhoods of the layout's tiles, for the passes that form a tile's gradients themselves. A
+// tile's local cells are its own cells [0, nct), its first ring [nct, nct + n1) (the cells of other
+// tiles that share a face with one of its cells), its second ring [.., nct + nr) (the further face
+// neighbours of the first ring) and a ghost for each boundary face of an own or first-ring cell.
+struct TileRings {
+    bool ok = false;             // false: a tile has more local cells than 16-bit indices hold
+    int max_local = 0;           // most local cells of a tile
+    int max_grad = 0;            // most own and first-ring cells of a tile (those with gradients)
+    std::vector<int> tiles;      // [4*ntiles] {ring start, n1 | ghosts << 16, nr, ghost start}
+    std::vector<int> cell;       // ring cells of the tiles in turn (renumbered), first then second ring
+    std::vector<uint16_t> own;   // [4*nc] local neighbours of each cell in its own tile, face order; 0xFFFF = none
+    std::vector<uint16_t> ring;  // [4*ring cells] the same of the first-ring cells (second ring unused)
+    std::vector<int> ghost;      // [2*ghosts] {owner (renumbered), face kind}
+    std::vector<double> ghost_n; // [2*ghosts] outward unit normal
+    std::vector<uint16_t> face;  // [2*face entries] local cells of L and R (R: the ghost on a boundary face)
+};
+void tile_rings(const RefMesh &m, const Layout &L, TileRings &r);
+
+// Per cell and face slot, renumbered cells: the least-squares vector (w, 8 doubles per cell), and
+// the outward unit normal and length (n, 12 doubles per cell); zero for unused slots.
+void cell_face_vectors(const Layout &L, std::vector<double> &w);
+void cell_face_normals(const Layout &L, std::vector<double> &n);
+
+// Centre offsets of the face entries, {dx, dy} each.
+void face_offsets(const Layout &L, std::vector<double> &d);
 
 // WENO line stencils of the layout's face entries: st gets 4 renumbered cells per entry,
 // {L-1, L-2, R+1, R+2}, where L-1 is the neighbour of L across the face opposite the entry's face
