@@ -3,8 +3,10 @@
 // accumulation, trained with Adam on FP32 master weights. Its prediction initialises the FP64
 // pseudo-time march of the plain solver.
 //
-// Device buffers per layer l (inputs K_l, outputs M_l, both padded to multiples of 32; rows of
-// a minibatch padded to a multiple of 512):
+// Networks of up to 256 padded features a layer train and predict through mlp_rows.hip (`rows`): per
+// layer only Xt_l and dZt_l, and the hidden layers' bf16 pre-activations, go through memory. Wider
+// ones go layer by layer (mlp_kernels.hip), with these buffers per layer l (inputs K_l, outputs M_l,
+// both padded to multiples of 32; rows of a minibatch padded to a multiple of 512):
 //   X_l  bf16 [rows x K_l] and its transpose Xt_l [K_l x rows]  (X_{l+1} = silu(Z_l))
 //   Z_l  fp32 [rows x M_l] pre-activations, dZ_l / dZt_l bf16 gradients
 //   W_l  fp32 master [M_l x K_l] (unpadded), bf16 copies Wb_l [M_l x K_l] and Wt_l [K_l x M_l]
@@ -55,6 +57,9 @@ struct cfd_mlp_s {
     float *Zo = nullptr;            // fp32 outputs of the last layer
     float *part = nullptr;          // split-K partials of every layer's weight gradient
     cfd::MlpLayers tab{};           // shapes and buffers of all layers, for the all-layer launches
+    bool rows = false;              // the network fits mlp_rows.hip
+    uint16_t *Zs = nullptr;         // its hidden pre-activations
+    float *pin = nullptr, *pout = nullptr;  // a chunk's features and predictions
     float *norm = nullptr;  // in_mean[n_in], in_scale[n_in], out_mean[n_out], out_scale[n_out]
     std::vector<float> norm_h;
     float *feat = nullptr, *targ = nullptr, *lrow = nullptr;
@@ -107,9 +112,12 @@ int forward(cfd_mlp_s *m, int rows) {
     return 0;
 }
 
+// Row ranges that the weight gradients are split over.
+int row_split(int rows) { return (rows % (32 * kSplitWide) == 0) ? kSplitWide : kSplit; }
+
 // Backward from dZ[L-1]/dZt[L-1] (set by the loss kernel); weight and bias gradients into gW, gb.
 int backward(cfd_mlp_s *m, int rows) {
-    const int split = (rows % (32 * kSplitWide) == 0) ? kSplitWide : kSplit;
+    const int split = row_split(rows);
     for (int l = m->L - 1; l >= 0; l--) {
         // dW_l = dZ_l^T X_l: A = dZt_l [Mp x rows], B = Xt_l [Kp x rows], split over rows
         MHIP(mlp_gemm(MLP_EPI_PARTIAL, m->dZt[l], rows, m->Xt[l], rows, m->Mp[l], m->Kp[l], rows, split,
@@ -125,6 +133,35 @@ int backward(cfd_mlp_s *m, int rows) {
     // launch each
     MHIP(mlp_reduce_layers(m->part, split, m->tab, m->gW, m->stream));
     MHIP(mlp_row_sum_layers(m->tab, rows, m->gb, m->stream));
+    return 0;
+}
+
+// Forward and backward of a minibatch of samples of m->feat and m->targ (drawn from (seed, step), or
+// the first rows in order), then the weight gradients' partial sums. With d_step, the step is *d_step
+// and advances.
+int rows_gradients(cfd_mlp_s *m, int n, int rows, bool draw, unsigned long long seed, int step, int *d_step) {
+    MlpRows a{};
+    a.feat = m->feat;
+    a.targ = m->targ;
+    a.norm = m->norm;
+    a.b = m->b;
+    a.n_in = m->n_in;
+    a.n_out = m->n_out;
+    a.n = n;
+    a.rows = rows;
+    a.draw = draw;
+    a.seed = seed;
+    a.step = step;
+    a.d_step = d_step;
+    a.Z = m->Zs;
+    a.lrow = m->lrow;
+    MHIP(mlp_rows(m->tab, a, true, m->stream));
+    MHIP(mlp_wgrad(m->tab, rows, row_split(rows), m->part, d_step, m->stream));
+    return 0;
+}
+
+int rows_update(cfd_mlp_s *m, int rows, const MlpAdam *a) {
+    MHIP(mlp_update(m->tab, m->part, row_split(rows), rows, a, m->gW, m->gb, m->stream));
     return 0;
 }
 
@@ -178,13 +215,19 @@ int cfd_mlp_create(int n_in, int width, int depth, int n_out, int max_rows, unsi
     }
     hipError_t e = hipSuccess;
     const int R = m->max_rows;
-    int maxMK = 0;
+    m->tab.L = m->L;
     size_t sumMK = 0;
     for (int l = 0; l < m->L; l++) {
-        maxMK = std::max(maxMK, m->Mp[l] * m->Kp[l]);
+        m->tab.M[l] = m->Mv[l];
+        m->tab.K[l] = m->Kv[l];
+        m->tab.Mp[l] = m->Mp[l];
+        m->tab.Kp[l] = m->Kp[l];
+        m->tab.woff[l] = (long long)m->woff[l];
+        m->tab.boff[l] = (long long)m->boff[l];
         m->tab.poff[l] = (long long)(kSplitWide * sumMK);
         sumMK += (size_t)m->Mp[l] * m->Kp[l];
     }
+    m->rows = m->tab.blocks = mlp_rows_fits(m->tab);
     bool ok = (e = m->alloc(&m->W, m->nw)) == hipSuccess && (e = m->alloc(&m->b, m->nb)) == hipSuccess &&
               (e = m->alloc(&m->mW, m->nw)) == hipSuccess && (e = m->alloc(&m->vW, m->nw)) == hipSuccess &&
               (e = m->alloc(&m->mb, m->nb)) == hipSuccess && (e = m->alloc(&m->vb, m->nb)) == hipSuccess &&
@@ -203,25 +246,22 @@ int cfd_mlp_create(int n_in, int width, int depth, int n_out, int max_rows, unsi
     for (int l = 0; ok && l < m->L; l++) {
         const size_t mk = (size_t)m->Mp[l] * m->Kp[l];
         ok = (e = m->alloc(&m->Wb[l], mk)) == hipSuccess && (e = m->alloc(&m->Wt[l], mk)) == hipSuccess &&
-             (e = m->alloc(&m->X[l], (size_t)R * m->Kp[l])) == hipSuccess &&
              (e = m->alloc(&m->Xt[l], (size_t)R * m->Kp[l])) == hipSuccess &&
-             (e = (l < m->L - 1 ? m->alloc(&m->Zh[l], (size_t)R * m->Mp[l])
-                                : m->alloc(&m->Zo, (size_t)R * m->Mp[l]))) == hipSuccess &&
-             (e = m->alloc(&m->dZ[l], (size_t)R * m->Mp[l])) == hipSuccess &&
              (e = m->alloc(&m->dZt[l], (size_t)R * m->Mp[l])) == hipSuccess;
-    }
-    m->tab.L = m->L;
-    for (int l = 0; ok && l < m->L; l++) {
-        m->tab.M[l] = m->Mv[l];
-        m->tab.K[l] = m->Kv[l];
-        m->tab.Mp[l] = m->Mp[l];
-        m->tab.Kp[l] = m->Kp[l];
-        m->tab.woff[l] = (long long)m->woff[l];
-        m->tab.boff[l] = (long long)m->boff[l];
+        if (ok && !m->rows)
+            ok = (e = m->alloc(&m->X[l], (size_t)R * m->Kp[l])) == hipSuccess &&
+                 (e = (l < m->L - 1 ? m->alloc(&m->Zh[l], (size_t)R * m->Mp[l])
+                                    : m->alloc(&m->Zo, (size_t)R * m->Mp[l]))) == hipSuccess &&
+                 (e = m->alloc(&m->dZ[l], (size_t)R * m->Mp[l])) == hipSuccess;
         m->tab.Wb[l] = m->Wb[l];
         m->tab.Wt[l] = m->Wt[l];
+        m->tab.Xt[l] = m->Xt[l];
         m->tab.dZt[l] = m->dZt[l];
     }
+    if (ok && m->rows)
+        ok = (e = m->alloc(&m->Zs, (size_t)(m->L - 1) * R * kMlpRowsWidth)) == hipSuccess &&
+             (e = m->alloc(&m->pin, (size_t)R * n_in)) == hipSuccess &&
+             (e = m->alloc(&m->pout, (size_t)R * n_out)) == hipSuccess;
     if (ok) e = hipStreamCreate(&m->stream);
     if (!ok || e != hipSuccess) {
         delete m;
@@ -303,14 +343,18 @@ int cfd_mlp_gradients(cfd_mlp_t *m, const float *feat, const float *targ, int n,
         return capi_fail(CFD_E_ARG, "cfd_mlp_gradients: n must be a positive multiple of 512 within max_rows");
     int rc = upload_data(m, feat, targ, n);
     if (rc) return rc;
-    MHIP(mlp_encode(m->feat, m->n_in, nullptr, n, nrm(m, 0), nrm(m, 1), m->Kp[0], m->X[0], m->Xt[0], n, m->stream));
-    rc = forward(m, n);
-    if (rc) return rc;
-    const int Lm = m->L - 1;
-    MHIP(mlp_loss(m->Zo, m->Mp[Lm], m->targ, m->n_out, nullptr, n, nrm(m, 2), nrm(m, 3), m->dZ[Lm], m->dZt[Lm], n,
-                  m->lrow, m->stream));
-    rc = backward(m, n);
-    if (rc) return rc;
+    if (m->rows) {
+        if ((rc = rows_gradients(m, n, n, false, 0, 0, nullptr)) || (rc = rows_update(m, n, nullptr))) return rc;
+    } else {
+        MHIP(mlp_encode(m->feat, m->n_in, nullptr, n, nrm(m, 0), nrm(m, 1), m->Kp[0], m->X[0], m->Xt[0], n, m->stream));
+        rc = forward(m, n);
+        if (rc) return rc;
+        const int Lm = m->L - 1;
+        MHIP(mlp_loss(m->Zo, m->Mp[Lm], m->targ, m->n_out, nullptr, n, nrm(m, 2), nrm(m, 3), m->dZ[Lm], m->dZt[Lm], n,
+                      m->lrow, m->stream));
+        rc = backward(m, n);
+        if (rc) return rc;
+    }
     MHIP(hipStreamSynchronize(m->stream));
     if (gW) MHIP(hipMemcpy(gW, m->gW, m->nw * sizeof(float), hipMemcpyDeviceToHost));
     if (gb) MHIP(hipMemcpy(gb, m->gb, m->nb * sizeof(float), hipMemcpyDeviceToHost));
@@ -343,6 +387,7 @@ int cfd_mlp_train(cfd_mlp_t *m, const float *feat, const float *targ, int n, int
         sch[3 * (size_t)s + 1] = 1.0f / (1.0f - std::pow(b1, (float)t));
         sch[3 * (size_t)s + 2] = 1.0f / (1.0f - std::pow(b2, (float)t));
     }
+    MlpAdam ad{m->W, m->mW, m->vW, m->b, m->mb, m->vb, 0.f, 0.f, 0.f, b1, b2, eps, nullptr, nullptr};
     auto log_loss = [&](int s) -> int {
         if (loss_hist && s % log_every == 0) {
             MHIP(hipMemcpyAsync(lrow.data(), m->lrow, batch * sizeof(float), hipMemcpyDeviceToHost, m->stream));
@@ -365,7 +410,13 @@ int cfd_mlp_train(cfd_mlp_t *m, const float *feat, const float *targ, int n, int
         MHIP(hipMemcpy(m->sched, sch.data(), 3 * (size_t)steps * sizeof(float), hipMemcpyHostToDevice));
         const int zero = 0;
         MHIP(hipMemcpy(m->d_step, &zero, sizeof(int), hipMemcpyHostToDevice));
+        ad.sched = m->sched;
+        ad.d_step = m->d_step;
         auto launches = [&]() -> int {
+            if (m->rows) {
+                if (int r = rows_gradients(m, n, batch, true, seed, 0, m->d_step)) return r;
+                return rows_update(m, batch, &ad);
+            }
             MHIP(mlp_sample_dev(seed, m->d_step, batch, n, m->idx, m->stream));
             MHIP(mlp_encode(m->feat, m->n_in, m->idx, batch, nrm(m, 0), nrm(m, 1), m->Kp[0], m->X[0], m->Xt[0],
                             batch, m->stream));
@@ -404,6 +455,16 @@ int cfd_mlp_train(cfd_mlp_t *m, const float *feat, const float *targ, int n, int
         return 0;
     }
     for (int s = 0; s < steps; s++) {
+        const float lrs = sch[3 * (size_t)s], c1 = sch[3 * (size_t)s + 1], c2 = sch[3 * (size_t)s + 2];
+        if (m->rows) {
+            ad.lr = lrs;
+            ad.c1 = c1;
+            ad.c2 = c2;
+            if ((rc = rows_gradients(m, n, batch, true, seed, s, nullptr)) || (rc = rows_update(m, batch, &ad))) return rc;
+            m->adam_t++;
+            if ((rc = log_loss(s))) return rc;
+            continue;
+        }
         MHIP(mlp_sample(seed, s, batch, n, m->idx, m->stream));
         MHIP(mlp_encode(m->feat, m->n_in, m->idx, batch, nrm(m, 0), nrm(m, 1), m->Kp[0], m->X[0], m->Xt[0], batch,
                         m->stream));
@@ -414,7 +475,6 @@ int cfd_mlp_train(cfd_mlp_t *m, const float *feat, const float *targ, int n, int
         rc = backward(m, batch);
         if (rc) return rc;
         m->adam_t++;
-        const float lrs = sch[3 * (size_t)s], c1 = sch[3 * (size_t)s + 1], c2 = sch[3 * (size_t)s + 2];
         MHIP(mlp_adam2(m->W, m->mW, m->vW, m->gW, (int)m->nw, m->b, m->mb, m->vb, m->gb, (int)m->nb, lrs, b1, b2,
                        eps, c1, c2, m->stream));
         rc = pack_all(m);
@@ -433,6 +493,25 @@ int cfd_mlp_set_launch(cfd_mlp_t *m, int mode) {
 
 int cfd_mlp_predict(cfd_mlp_t *m, const float *feat, int n, float *out) {
     if (!m || !feat || !out || n <= 0) return capi_fail(CFD_E_ARG, "cfd_mlp_predict: bad arguments");
+    if (m->rows) {
+        for (int r0 = 0; r0 < n; r0 += m->max_rows) {
+            MlpRows a{};
+            a.n = std::min(m->max_rows, n - r0);
+            a.feat = m->pin;
+            a.norm = m->norm;
+            a.b = m->b;
+            a.n_in = m->n_in;
+            a.n_out = m->n_out;
+            a.out = m->pout;
+            MHIP(hipMemcpyAsync(m->pin, feat + (size_t)r0 * m->n_in, (size_t)a.n * m->n_in * sizeof(float),
+                                hipMemcpyHostToDevice, m->stream));
+            MHIP(mlp_rows(m->tab, a, false, m->stream));
+            MHIP(hipMemcpyAsync(out + (size_t)r0 * m->n_out, m->pout, (size_t)a.n * m->n_out * sizeof(float),
+                                hipMemcpyDeviceToHost, m->stream));
+        }
+        MHIP(hipStreamSynchronize(m->stream));
+        return 0;
+    }
     const int Lm = m->L - 1, C = m->Mp[Lm];
     std::vector<float> z((size_t)m->max_rows * C);
     const float *om = m->norm_h.data() + 2 * m->n_in, *os = om + m->n_out;
@@ -465,6 +544,12 @@ int cfd_mlp_time_step(cfd_mlp_t *m, int batch, int reps, float *ms) {
     MHIP(hipEventCreate(&e1));
     MHIP(hipEventRecord(e0, m->stream));
     for (int s = 0; s < reps; s++) {
+        if (m->rows) {
+            int rc = rows_gradients(m, (int)m->data_cap, batch, true, 7, s, nullptr);
+            if (!rc) rc = rows_update(m, batch, nullptr);
+            if (rc) return rc;
+            continue;
+        }
         MHIP(mlp_sample(7, s, batch, (int)m->data_cap, m->idx, m->stream));
         MHIP(mlp_encode(m->feat, m->n_in, m->idx, batch, nrm(m, 0), nrm(m, 1), m->Kp[0], m->X[0], m->Xt[0], batch,
                         m->stream));

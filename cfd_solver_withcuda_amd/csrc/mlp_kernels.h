@@ -14,9 +14,40 @@ struct MlpLayers {
     int L;
     int M[kMlpMaxLayers], K[kMlpMaxLayers], Mp[kMlpMaxLayers], Kp[kMlpMaxLayers];
     long long woff[kMlpMaxLayers], boff[kMlpMaxLayers], poff[kMlpMaxLayers];
-    uint16_t *Wb[kMlpMaxLayers], *Wt[kMlpMaxLayers];
-    const uint16_t *dZt[kMlpMaxLayers];
+    uint16_t *Wb[kMlpMaxLayers], *Wt[kMlpMaxLayers];  // bf16 weights and their transposes
+    bool blocks;                                       // Wb, Wt in MFMA operand order (mlp_rows), else row-major
+    uint16_t *Xt[kMlpMaxLayers], *dZt[kMlpMaxLayers];  // transposed inputs and gradients: [features x rows],
+                                                       // of mlp_rows [rows / 32][features][32]
 };
+
+// ---- networks of up to kMlpRowsWidth padded features a layer (mlp_rows.hip) -------------------
+constexpr int kMlpRowsWidth = 256;
+struct MlpRows {
+    const float *feat, *targ, *norm, *b;  // samples [n]; normalisation (mean, scale of in, then out); biases
+    int n_in, n_out, n, rows;             // samples, minibatch rows (training)
+    int draw, step;                       // draw the rows' samples from (seed, step), else row r is sample r
+    unsigned long long seed;
+    const int *d_step;                    // the step in device memory (captured sequences)
+    uint16_t *Z;                          // bf16 pre-activations of the hidden layers [L - 1][rows x 256]
+    float *lrow;                          // per-row loss
+    float *out;                           // predictions [n x n_out], physical units
+};
+struct MlpAdam {
+    float *W, *mW, *vW, *b, *mb, *vb;
+    float lr, c1, c2, b1, b2, eps;
+    const float *sched;  // with d_step: the rates of step *d_step - 1
+    const int *d_step;
+};
+bool mlp_rows_fits(const MlpLayers &t);
+// Training: forward and backward of the minibatch (t.Xt, t.dZt, a.Z, a.lrow); else predictions.
+hipError_t mlp_rows(const MlpLayers &t, const MlpRows &a, bool train, hipStream_t s);
+// Weight gradients of all layers over `split` row ranges into P (as mlp_reduce_layers reads them);
+// *d_step += 1 when given.
+hipError_t mlp_wgrad(const MlpLayers &t, int rows, int split, float *P, int *d_step, hipStream_t s);
+// Sums over the ranges and of the biases' rows, then Adam with the bf16 copies (a), or the gradients
+// alone (a = null).
+hipError_t mlp_update(const MlpLayers &t, const float *P, int split, int rows, const MlpAdam *a, float *gW, float *gb,
+                      hipStream_t s);
 
 // C[r][c] = sum_k A[r][k] B[c][k] (bf16 in, fp32 accumulate) with the epilogue `epi`:
 //   BIAS_SILU: Zout = C + bias (bf16 pre-activations, ld C), Y = silu(C + bias) (bf16, ld ldy),

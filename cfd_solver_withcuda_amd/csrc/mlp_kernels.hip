@@ -15,28 +15,11 @@
 
 #include <algorithm>
 
+#include "mlp_device.h"
 #include "mlp_kernels.h"
 
 namespace cfd {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// round-to-nearest-even float -> bf16 bits
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (uint16_t)((u >> 16) | ((u & 0xffff) ? 0x40 : 0));  // inf / nan
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-
-__device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + __expf(-z)); }
-
-__device__ __forceinline__ bf16x8 load8(const uint16_t *p) {
-    return *reinterpret_cast<const bf16x8 *>(p);
-}
 
 // Epilogues
 enum { EPI_BIAS_SILU = MLP_EPI_BIAS_SILU, EPI_BIAS = MLP_EPI_BIAS, EPI_DSILU = MLP_EPI_DSILU, EPI_PARTIAL = MLP_EPI_PARTIAL };
@@ -361,11 +344,7 @@ __global__ void __launch_bounds__(256) sample_kernel(unsigned long long seed, in
                                                      int n, int *__restrict__ idx) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
-    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * ((unsigned long long)step * (unsigned long long)rows + r + 1);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    idx[r] = (int)(z % (unsigned long long)n);
+    idx[r] = sample_index(seed, step, rows, r, n);
 }
 
 // The minibatch of a captured training step's step *d_step (the step's Adam reads its rates
@@ -374,27 +353,11 @@ __global__ void __launch_bounds__(256) sample_dev_kernel(unsigned long long seed
                                                          int rows, int n, int *__restrict__ idx) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
-    const int step = *d_step;
-    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * ((unsigned long long)step * (unsigned long long)rows + r + 1);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    idx[r] = (int)(z % (unsigned long long)n);
+    idx[r] = sample_index(seed, *d_step, rows, r, n);
 }
 
 
 // ---- all layers in one launch ---------------------------------------------------------------
-// One Adam element update: moments m1, m2 and W -= lr (m1 c1) / (sqrt(m2 c2) + eps).
-__device__ __forceinline__ void adam_one(float *W, float *m1, float *m2, const float *g, int i, float lr,
-                                         float b1, float b2, float eps, float c1, float c2) {
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.0f - b1) * gi;
-    const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = b;
-    W[i] -= lr * (a * c1) / (sqrtf(b * c2) + eps);
-}
-
 // Adam over weights [0, nw) and biases [nw, nw + nb) in one grid; with d_step the step's rates
 // are sched[3 step .. 3 step + 2], else lr, c1, c2.
 __global__ void __launch_bounds__(256) adam2_kernel(float *__restrict__ W, float *__restrict__ mW,
@@ -413,8 +376,8 @@ __global__ void __launch_bounds__(256) adam2_kernel(float *__restrict__ W, float
         c1 = sched[3 * step + 1];
         c2 = sched[3 * step + 2];
     }
-    if (i < nw) adam_one(W, mW, vW, gW, i, lr, b1, b2, eps, c1, c2);
-    else adam_one(b, mb, vb, gb, i - nw, lr, b1, b2, eps, c1, c2);
+    if (i < nw) adam_one(W[i], mW[i], vW[i], gW[i], lr, b1, b2, eps, c1, c2);
+    else adam_one(b[i - nw], mb[i - nw], vb[i - nw], gb[i - nw], lr, b1, b2, eps, c1, c2);
 }
 
 // W -> Wb [Mp x Kp] and Wt [Kp x Mp] (bf16, zero padding) of layer blockIdx.y; block (0, 0) also
@@ -427,8 +390,8 @@ __global__ void __launch_bounds__(256) pack_layers_kernel(const float *__restric
     if (i >= Mp * Kp) return;
     const int m = i / Kp, k = i % Kp;
     const uint16_t h = (m < M && k < K) ? f2bf(W[t.woff[l] + (size_t)m * K + k]) : (uint16_t)0;
-    t.Wb[l][i] = h;
-    t.Wt[l][(size_t)k * Mp + m] = h;
+    t.Wb[l][t.blocks ? operand_at(m, k, Kp) : i] = h;
+    t.Wt[l][t.blocks ? operand_at(k, m, Mp) : (size_t)k * Mp + m] = h;
 }
 
 // Split-K partial sums of layer blockIdx.y, in split order, into its unpadded gradient.
@@ -446,33 +409,16 @@ __global__ void __launch_bounds__(256) reduce_layers_kernel(const float *__restr
     gW[t.woff[l] + i] = s;
 }
 
-// Bias gradients of every layer: block b is row b of the layers' rows in turn; eight values per
-// thread and step (one 16-byte load), four steps in flight (n a multiple of 512), the partial sums
-// combined in a fixed order.
+// Bias gradients of every layer: block b is row b of the layers' rows in turn. The 256 parts of a row
+// are combined in a fixed order.
 __global__ void __launch_bounds__(256) row_sum_layers_kernel(MlpLayers t, int n, float *__restrict__ gb) {
-    __shared__ float red[256];
     int r = blockIdx.x, l = 0;
     while (l < t.L - 1 && r >= t.M[l]) r -= t.M[l++];
-    const int tt = threadIdx.x;
     const uint16_t *row = t.dZt[l] + (size_t)r * n;
+    __shared__ float red[256];
+    const int tt = threadIdx.x;
     float s4[4] = {0.f, 0.f, 0.f, 0.f};
-    int j = 8 * tt;
-    for (; j + 3 * 2048 < n; j += 4 * 2048)
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const uint4 v = *reinterpret_cast<const uint4 *>(row + j + u * 2048);
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int q = 0; q < 4; q++) s4[u] += bf2f((uint16_t)(w[q] & 0xffff)) + bf2f((uint16_t)(w[q] >> 16));
-        }
-    for (; j < n; j += 2048) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(row + j);
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int q = 0; q < 4; q++) s4[0] += bf2f((uint16_t)(w[q] & 0xffff)) + bf2f((uint16_t)(w[q] >> 16));
-    }
-    const float sum = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-    red[tt] = sum;
+    red[tt] = row_part([&](int j) { return row + j; }, 8 * tt, n, s4);
     __syncthreads();
     for (int h = 128; h > 0; h >>= 1) {
         if (tt < h) red[tt] += red[tt + h];
@@ -480,7 +426,6 @@ __global__ void __launch_bounds__(256) row_sum_layers_kernel(MlpLayers t, int n,
     }
     if (tt == 0) gb[t.boff[l] + r] = red[0];
 }
-
 
 }  // namespace
 
