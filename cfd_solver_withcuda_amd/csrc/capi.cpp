@@ -517,7 +517,8 @@ static int ensure_ref_cells(cfd_mesh_s *m) {
 
 // The reference's Evaluate_Cell_Net_Flux_2O (Roe on limited differences): physical state and
 // ghosts (exit ghosts from uexit when set) gathered into Uall, then the cell-by-cell kernel.
-static int ref_roe2o_pass(cfd_solver_s *s, const double4 *in, double *dtmin, const double4 *uexit, hipStream_t st) {
+static bool ref_roe2o(const cfd_config_t &c) { return c.ref_mode && c.order == 2 && c.flux == FLUX_ROE; }
+static int ref_roe2o_pass(cfd_solver_s *s, const double4 *in, bool want_min, const double4 *uexit, hipStream_t st) {
     cfd_mesh_s *m = s->m;
     const int nc = m->ref.nc, ng = m->ref.ng;
     int rc = ensure_ref_cells(m);
@@ -528,8 +529,7 @@ static int ref_roe2o_pass(cfd_solver_s *s, const double4 *in, double *dtmin, con
                           uexit, s->Uall + nc, st));
     const RefCells cells{m->d_rc_nf, m->d_rc_nbr, m->d_rc_dist, m->d_rc_nrm, m->d_rc_len, m->d_rc_area};
     HIP_TRY(launch_roe2o(nc, cells, s->Uall, s->cfg.zeta, s->cfg.zeta1, s->cfg.cfl, s->R, s->dt,
-                         dtmin ? s->dt_partial : nullptr, st));
-    if (dtmin) HIP_TRY(launch_min_reduce(s->dt_partial, (nc + 255) / 256, dtmin, st));
+                         want_min ? s->dt_partial : nullptr, st));
     return 0;
 }
 
@@ -537,21 +537,26 @@ static int ref_roe2o_pass(cfd_solver_s *s, const double4 *in, double *dtmin, con
 // depend on the order, so a first-order pass suffices; the viscous term exists at order 2 only.
 static int dt_pass_order(const cfd_config_t &c) { return c.viscous ? 2 : 1; }
 
-// residual of state `in` into s->R, s->dt (+ minimum dt into *dtmin when set)
+// residual of state `in` into s->R, s->dt (+ partial minima of dt into s->dt_partial, + their minimum
+// into *dtmin when set)
 static int residual_pass(cfd_solver_s *s, const double4 *in, double *dtmin, const double4 *uexit,
-                         hipStream_t st, int order_override = 0, bool want_grad = false) {
+                         hipStream_t st, int order_override = 0, bool want_grad = false, bool partials = false) {
     const cfd_config_t &c = s->cfg;
     const int order = order_override ? order_override : c.order;
-    if (c.ref_mode && order == 2 && c.flux == FLUX_ROE) return ref_roe2o_pass(s, in, dtmin, uexit, st);
-    StageArgs a = resid_args(s, dtmin != nullptr, uexit);
-    if (order == 2) {
+    const bool want_min = dtmin || partials;
+    StageArgs a = resid_args(s, want_min, uexit);
+    int n = s->dev.ntiles;
+    if (order == c.order && ref_roe2o(c)) {
+        if (int rc = ref_roe2o_pass(s, in, want_min, uexit, st)) return rc;
+        n = (s->m->ref.nc + 255) / 256;
+    } else if (order == 2) {
         HIP_TRY(launch_second_order(s->dev, s->dcfg, c.flux, c.limiter, c.gradient, MODE_RESID, in, s->grad, want_grad,
                                     a, 0, c.block, st));
     } else {
         if (order == 3) HIP_TRY(launch_grad(s->dev, s->dcfg, c.gradient, in, s->grad, c.block, st));
         HIP_TRY(launch_flux(s->dev, s->dcfg, c.flux, order, c.limiter, MODE_RESID, in, s->grad, a, c.block, st));
     }
-    if (dtmin) HIP_TRY(launch_min_reduce(s->dt_partial, s->dev.ntiles, dtmin, st));
+    if (dtmin) HIP_TRY(launch_min_reduce(s->dt_partial, n, dtmin, st));
     return 0;
 }
 
@@ -722,26 +727,29 @@ static int native_step(cfd_solver_s *s, bool want_err, hipStream_t st) {
     return 0;
 }
 
-// One iteration of the reference's Inviscid_Solver loop body.
-static int ref_step(cfd_solver_s *s, hipStream_t st) {
+// One iteration of the reference's Inviscid_Solver loop body. Where the time step's partial minima are
+// few, every workgroup of the update takes their minimum itself: a launch less per stage. (Above that
+// the workgroups' reads, partials x cells / 256, would cost more than the launch.)
+static int ref_step(cfd_solver_s *s, bool want_err, hipStream_t st) {
     const cfd_config_t &c = s->cfg;
     const int nc = s->m->ref.nc;
     const int nb = (nc + 255) / 256;
+    const int np = ref_roe2o(c) ? nb : s->dev.ntiles;
+    const bool own = np <= 1024;
     double *dmin = s->scal + 2;
-    const double4 *R = s->R;
+    auto stage = [&](int kind, const double4 *in, double4 *out) -> int {
+        if (int rc = residual_pass(s, in, own ? nullptr : dmin, s->Un, st, 0, false, own)) return rc;
+        HIP_TRY(launch_ref_update(nc, kind, kind == 0 && c.lts, s->m->d_inv_area, s->Un, in, s->R, s->dt, s->dt_partial,
+                                  own ? np : 0, dmin, out, kind >= 2 && want_err ? s->err_partial : nullptr, st));
+        return 0;
+    };
     int rc;
     if (c.rk == 1) {
-        if ((rc = residual_pass(s, s->Un, dmin, s->Un, st))) return rc;
-        HIP_TRY(launch_ref_update(nc, 3, 0, s->m->d_inv_area, s->Un, s->Un, R, s->dt, dmin, s->Un, s->err_partial, st));
-    } else {
-        if ((rc = residual_pass(s, s->Un, dmin, s->Un, st))) return rc;
-        HIP_TRY(launch_ref_update(nc, 0, c.lts, s->m->d_inv_area, s->Un, s->Un, R, s->dt, dmin, s->Ua, nullptr, st));
-        if ((rc = residual_pass(s, s->Ua, dmin, s->Un, st))) return rc;
-        HIP_TRY(launch_ref_update(nc, 1, 0, s->m->d_inv_area, s->Un, s->Ua, R, s->dt, dmin, s->Ub, nullptr, st));
-        if ((rc = residual_pass(s, s->Ub, dmin, s->Un, st))) return rc;
-        HIP_TRY(launch_ref_update(nc, 2, 0, s->m->d_inv_area, s->Un, s->Ub, R, s->dt, dmin, s->Un, s->err_partial, st));
+        if ((rc = stage(3, s->Un, s->Un))) return rc;
+    } else if ((rc = stage(0, s->Un, s->Ua)) || (rc = stage(1, s->Ua, s->Ub)) || (rc = stage(2, s->Ub, s->Un))) {
+        return rc;
     }
-    HIP_TRY(launch_err_finalize(s->err_partial, nb, s->scal + 3, st));
+    if (want_err) HIP_TRY(launch_err_finalize(s->err_partial, nb, s->scal + 3, st));
     return 0;
 }
 
@@ -753,7 +761,7 @@ int cfd_step(cfd_solver_t *s, int nsteps, double *err_hist, double *dt_hist, voi
     const bool sync = err_hist || dt_hist;
     for (int n = 0; n < nsteps; n++) {
         const int cur_before = s->cur;
-        int rc = s->cfg.ref_mode ? ref_step(s, st) : native_step(s, err_hist != nullptr, st);
+        int rc = s->cfg.ref_mode ? ref_step(s, err_hist != nullptr, st) : native_step(s, err_hist != nullptr, st);
         if (rc) return rc;
         if (sync) {
             double h[8];
@@ -849,7 +857,7 @@ int cfd_run_steady(cfd_solver_t *s, double tol, int max_steps, int check_every, 
         const int chunk = std::min(check_every, max_steps - done);
         for (int n = 0; n < chunk; n++) {
             const bool want = (n == chunk - 1);
-            int rc = s->cfg.ref_mode ? ref_step(s, st) : native_step(s, want, st);
+            int rc = s->cfg.ref_mode ? ref_step(s, want, st) : native_step(s, want, st);
             if (rc) return rc;
             if (!s->cfg.ref_mode && !s->cfg.lts) s->cur = 1 - s->cur;
         }

@@ -113,7 +113,7 @@ hipError_t launch_roe2o(int nc, const RefCells &rc, const double4 *U_all, double
 hipError_t launch_min_reduce(const double *partial, int n, double *out, hipStream_t s);
 hipError_t launch_ref_update(int nc, int kind, int lts, const double *inv_area, const double4 *Un,
                              const double4 *Us, const double4 *R, const double *dt_cell,
-                             const double *dt_global, double4 *Uout, double *err_partial,
-                             hipStream_t s);
+                             const double *dt_partial, int npart, double *dt_global, double4 *Uout,
+                             double *err_partial, hipStream_t s);
 
 }  // namespace cfd

@@ -505,23 +505,43 @@ __global__ void __launch_bounds__(1024) min_reduce_kernel(const double *partial,
 // 342-457) with the stage's global dt (device scalar) and, in stage 0 with LTS, the cell's dt.
 // kind 0: U1 = Un - dt/A R; 1: U2 = 1/4 (U1 + 3 Un - dt/A R); 2: dU = 2/3 (U2 - Un - dt/A R),
 // Uout = Un + dU; 3 (forward Euler): dU = -dt/A R, Uout = Un + dU. Kinds 2 and 3 also emit the
-// error partials of dU.
+// error partials of dU where err_partial is given. The global dt is the minimum of the npart partials
+// (workgroup 0 writes it to *dt_global), or already there (npart 0).
 __global__ void __launch_bounds__(256) ref_update_kernel(int nc, int kind, int lts,
                                                          const double *__restrict__ inv_area,
                                                          const double4 *__restrict__ Un,
                                                          const double4 *__restrict__ Us,
                                                          const double4 *__restrict__ R,
                                                          const double *__restrict__ dt_cell,
-                                                         const double *__restrict__ dt_global,
+                                                         const double *__restrict__ dt_partial, int npart,
+                                                         double *__restrict__ dt_global,
                                                          double4 *__restrict__ Uout,
                                                          double *__restrict__ err_partial) {
     __shared__ double red[4 * 256];
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     double e[4] = {0, 0, 0, 0};
+    double ia = 0.0;
+    double4 n4{}, s4{}, r4{};
     if (c < nc) {
-        const double dtg = *dt_global;
-        const double ia = inv_area[c];
-        const double4 n4 = Un[c], s4 = Us[c], r4 = R[c];
+        ia = inv_area[c];
+        n4 = Un[c];
+        s4 = Us[c];
+        r4 = R[c];
+    }
+    double dtg;
+    if (npart) {
+        dtg = 1.7976931348623157e308;
+        for (int i = threadIdx.x; i < npart; i += 256) dtg = fmin(dtg, dt_partial[i]);
+        for (int d = 32; d > 0; d >>= 1) dtg = fmin(dtg, __shfl_xor(dtg, d));
+        if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = dtg;
+        __syncthreads();
+        dtg = fmin(fmin(red[0], red[1]), fmin(red[2], red[3]));
+        __syncthreads();  // red is the error's next
+        if (blockIdx.x == 0 && threadIdx.x == 0) *dt_global = dtg;
+    } else {
+        dtg = *dt_global;
+    }
+    if (c < nc) {
         const double un[4] = {n4.x, n4.y, n4.z, n4.w};
         const double us[4] = {s4.x, s4.y, s4.z, s4.w};
         const double r[4] = {r4.x, r4.y, r4.z, r4.w};
@@ -552,7 +572,7 @@ __global__ void __launch_bounds__(256) ref_update_kernel(int nc, int kind, int l
         }
         Uout[c] = make_double4(o[0], o[1], o[2], o[3]);
     }
-    if (kind >= 2) {
+    if (err_partial) {
         double out[4];
         block_sum4(red, e, out, blockDim.x);
         if (threadIdx.x == 0)
@@ -605,6 +625,8 @@ int persist_grid(const void *kernel, const DevMesh &m, const DevCfg &c, int bloc
     return std::min(g, full);
 }
 
+constexpr int kComputeUnits = 256;
+
 // LDS of one flux launch: the face-geometry copy (3 doubles per face) only when the launch forms
 // time steps (the kernel's needN), at least the block reductions' 4 doubles per thread.
 size_t flux_launch_smem(const DevMesh &m, int order, int grad_lds, int block, bool geom) {
@@ -619,6 +641,10 @@ hipError_t launch_flux(const DevMesh &m, const DevCfg &c, int flux, int order, i
                        const double4 *Us, const double *grad, const StageArgs &st, int block,
                        hipStream_t s) {
     const bool geom = (mode == MODE_RESID) || (st.lts && st.stage == 0) || (st.last && st.dt_partial);
+    // A residual of no more tiles than compute units takes as long as one tile's chain of arithmetic:
+    // the kernel's most threads for its faces (16k cells in tiles of 128: 8.65 -> 8.25 us). The results
+    // don't depend on the threads; a stage's error sums do.
+    if (mode == MODE_RESID && grid_of(m, c) <= kComputeUnits && m.max_tile_faces > block) block = 256;
     const size_t sm = flux_launch_smem(m, order, c.grad_lds, block, geom);
     if (c.persist) {
         if (mode != MODE_STAGE || order > 2 || c.viscous) return hipErrorInvalidValue;
@@ -643,7 +669,6 @@ bool fused_fits(const DevMesh &m, const DevCfg &c, int gradient, int block) {
 // units idle (no more tiles than compute units; the recomputing pass, of few tiles): there the time
 // is one tile's chain of arithmetic, and one thread per face shortens it.
 static int fused_threads(const DevMesh &m, const DevCfg &c, int block, int most, bool few) {
-    constexpr int kComputeUnits = 256;
     if (!few && grid_of(m, c) > kComputeUnits) return block;
     return std::max(block, std::min(most, (m.max_tile_faces + 63) / 64 * 64));
 }
@@ -746,11 +771,11 @@ hipError_t launch_min_reduce(const double *partial, int n, double *out, hipStrea
 
 hipError_t launch_ref_update(int nc, int kind, int lts, const double *inv_area, const double4 *Un,
                              const double4 *Us, const double4 *R, const double *dt_cell,
-                             const double *dt_global, double4 *Uout, double *err_partial,
-                             hipStream_t s) {
+                             const double *dt_partial, int npart, double *dt_global, double4 *Uout,
+                             double *err_partial, hipStream_t s) {
     if (nc <= 0) return hipSuccess;
     hipLaunchKernelGGL(ref_update_kernel, dim3((nc + 255) / 256), dim3(256), 0, s, nc, kind, lts,
-                       inv_area, Un, Us, R, dt_cell, dt_global, Uout, err_partial);
+                       inv_area, Un, Us, R, dt_cell, dt_partial, npart, dt_global, Uout, err_partial);
     return hipGetLastError();
 }
 
