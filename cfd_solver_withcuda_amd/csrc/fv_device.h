@@ -549,11 +549,50 @@ __device__ __forceinline__ double weno5(double a, double b, double c, double d, 
     return isfinite(U) ? U : c;
 }
 
-// Face state from WENO-reconstructed conserved values (Calculate_Primitive_Variables on U_L /
-// U_R, src/WENO2D.cpp:482-489); a non-positive density or pressure falls back to the cell state.
-__device__ __forceinline__ void weno_face_state(const double *U, const FState &cell, FState &out) {
-    state_from_U(U[0], U[1], U[2], U[3], out);
-    if (!(out.W[0] > 0.0) || !(out.W[3] > 0.0)) out = cell;
+// Quotients without the range handling (scaling and special cases) of the compiler's division: the
+// same reciprocal estimate, two steps of Newton's method and one residual step, so the same bits while
+// b and 1 / b are normal and the quotient is (compared over 10^9 random pairs); 8 instructions instead of
+// 11, and 3 for each further quotient of one b. Of WENO5's nine quotients per face value, all but one
+// branch's go this way: with one copy of the face code instead of three, 95 -> 70 us a stage of 405k
+// cells of the channel bump on MI355X.
+__device__ __forceinline__ double plain_rcp(double b) {
+    const double y0 = __builtin_amdgcn_rcp(b);
+    const double y1 = __builtin_fma(y0, __builtin_fma(-b, y0, 1.0), y0);
+    return __builtin_fma(y1, __builtin_fma(-b, y1, 1.0), y1);
+}
+// a / b with y = plain_rcp(b), or the rounded 1 / b of a constant. The residual is taken negated so that
+// -0 stays -0.
+__device__ __forceinline__ double plain_div(double a, double b, double y) {
+    const double q = a * y;
+    return __builtin_fma(-__builtin_fma(b, q, -a), y, q);
+}
+
+// The two face values of weno5 (a, b, c | d, e, f: left with shift 0, right with shift 1) for inputs
+// below 2^200, where every square and quotient of the weights is normal. A NaN among a value's inputs makes
+// it one.
+__device__ __forceinline__ void weno5_pair(double a, double b, double c, double d, double e, double f, double &UL,
+                                           double &UR) {
+    const double eps = 1e-6, y6 = 1.0 / 6.0;
+    auto smooth = [](double s, double t) { return (13.0 / 12.0) * (s * s) + (1.0 / 4.0) * (t * t); };
+    auto combine = [&](double d0, double d2, double b0, double b1, double b2, double v0, double v1, double v2) {
+        const double e0 = eps + b0, e1 = eps + b1, e2 = eps + b2;
+        const double q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
+        const double a0 = plain_div(d0, q0, plain_rcp(q0));
+        const double a1 = plain_div(6.0 / 10.0, q1, plain_rcp(q1));
+        const double a2 = plain_div(d2, q2, plain_rcp(q2));
+        const double sum = a0 + a1 + a2;
+        if (sum < eps) return (v0 + v1 + v2) / 3.0;
+        const double y = plain_rcp(sum);
+        return plain_div(a0, sum, y) * v0 + plain_div(a1, sum, y) * v1 + plain_div(a2, sum, y) * v2;
+    };
+    // second differences of the four stencils, left to right
+    const double s1 = a - 2.0 * b + c, s2 = b - 2.0 * c + d, s3 = c - 2.0 * d + e, s4 = d - 2.0 * e + f;
+    UL = combine(3.0 / 10.0, 1.0 / 10.0, smooth(s3, 3.0 * c - 4.0 * d + e), smooth(s2, b - d),
+                 smooth(s1, a - 4.0 * b + 3.0 * c), plain_div(2.0 * c + 5.0 * d - 1.0 * e, 6.0, y6),
+                 plain_div(-1.0 * b + 5.0 * c + 2.0 * d, 6.0, y6), plain_div(2.0 * a - 7.0 * b + 11.0 * c, 6.0, y6));
+    UR = combine(1.0 / 10.0, 3.0 / 10.0, smooth(s4, 3.0 * d - 4.0 * e + f), smooth(s3, c - e),
+                 smooth(s2, b - 4.0 * c + 3.0 * d), plain_div(11.0 * d - 7.0 * e + 2.0 * f, 6.0, y6),
+                 plain_div(2.0 * c + 5.0 * d - 1.0 * e, 6.0, y6), plain_div(-1.0 * b + 5.0 * c + 2.0 * d, 6.0, y6));
 }
 
 // ------------------------------------------------------------------------------------------

@@ -196,6 +196,60 @@ __device__ __forceinline__ void load_grad(const double *__restrict__ grad, int c
     }
 }
 
+// Face states by WENO5 on the conserved variables along the line of quadrilaterals through the face,
+// cells L-2, L-1, L | R, R+1, R+2 (st: L-1, L-2, R+1, R+2). The quotients of the weights go without range
+// handling where the inputs allow it, which is practically always.
+__device__ __forceinline__ void weno_line(int4 st, const double4 *__restrict__ Us, const double *sU, int T, int c0,
+                                          int nct, const FaceRec &f, FState &fL, FState &fR) {
+    const int cell[6] = {st.y, st.x, f.L, f.R, st.z, st.w};
+    double u[6][4], UL[4], UR[4];
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        const int l = cell[i] - c0;
+        if ((unsigned)l < (unsigned)nct) {
+            for (int q = 0; q < 4; q++) u[i][q] = sU[q * T + l];
+        } else {
+            const double4 v = Us[cell[i]];
+            u[i][0] = v.x;
+            u[i][1] = v.y;
+            u[i][2] = v.z;
+            u[i][3] = v.w;
+        }
+    }
+    double most = 0.0;
+    bool plain = true;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        for (int i = 0; i < 6; i++) most = fmax(most, fabs(u[i][q]));
+        weno5_pair(u[0][q], u[1][q], u[2][q], u[3][q], u[4][q], u[5][q], UL[q], UR[q]);
+        plain = plain && isfinite(UL[q]) && isfinite(UR[q]);
+    }
+    if (!(plain && most < 0x1p200)) {
+#pragma unroll 1
+        for (int q = 0; q < 4; q++) {
+            double v[6];
+            for (int i = 0; i < 6; i++) {
+                const int l = cell[i] - c0;
+                v[i] = (unsigned)l < (unsigned)nct ? sU[q * T + l] : reinterpret_cast<const double *>(Us + cell[i])[q];
+            }
+            const double l = weno5(v[0], v[1], v[2], v[3], v[4], 0), r = weno5(v[1], v[2], v[3], v[4], v[5], 1);
+            for (int i = 0; i < 4; i++)
+                if (i == q) {
+                    UL[i] = l;
+                    UR[i] = r;
+                }
+        }
+    }
+    // a non-positive density or pressure falls back to the cell's state (Calculate_Primitive_Variables
+    // on U_L / U_R, src/WENO2D.cpp:482-489)
+    auto state = [&](const double *U, int c, FState &out) {
+        state_from_U(U[0], U[1], U[2], U[3], out);
+        if (!(out.W[0] > 0.0) || !(out.W[3] > 0.0)) load_state(Us, c, out);
+    };
+    state(UL, f.L, fL);
+    state(UR, f.R, fR);
+}
+
 template <int FLUX, int ORDER, int LIM, bool VISC, int POS = 0>
 __device__ __forceinline__ void flux_face(const DevMesh &m, const DevCfg &cfg,
                                           const double4 *__restrict__ Us,
@@ -223,35 +277,39 @@ __device__ __forceinline__ void flux_face(const DevMesh &m, const DevCfg &cfg,
     }
     const int lL = f.L - c0;
     const bool locL = (unsigned)lL < (unsigned)nct;
-    FState SL, SR;
-    // Tile cells come from LDS: primitives always, conserved values at first order and for WENO
-    // (the MUSCL face states form their conserved values from the reconstructed primitives).
-    if (locL) {
-        for (int q = 0; q < 5; q++) SL.W[q] = sW[q * T + lL];
-        if constexpr (ORDER != 2)
-            for (int q = 0; q < 4; q++) SL.U[q] = sU[q * T + lL];
-    } else {
-        load_state(Us, f.L, SL);
-    }
     const bool boundary = f.R < 0;
-    int bc = 0;
-    bool locR = false;
-    int lR = 0;
-    if (boundary) {
-        bc = cfg.bc[-f.R];
-        // ghost of the cell-centre state (at second order only its primitives are used: the
-        // L side's reconstruction differences toward it)
-        if (bc == BC_EXIT && Uexit) {
-            FState src;
-            load_state(Uexit, f.L, src);
-            ghost_state(bc, src, nx, ny, fsv, SR);
+    const int bc = boundary ? cfg.bc[-f.R] : 0;
+    const int lR = boundary ? -1 : f.R - c0;
+    const bool locR = (unsigned)lR < (unsigned)nct;
+    FState SL, SR;  // of the cells
+    FState fL, fR;  // of the face
+    bool line = false;
+    if constexpr (ORDER == 3) {
+        const int4 st = boundary ? make_int4(-1, -1, -1, -1) : m.fst[e];
+        line = st.x >= 0;
+        if (line) weno_line(st, Us, sU, T, c0, nct, f, fL, fR);
+    }
+    if (!line || VISC) {
+        // Tile cells come from LDS: primitives always, conserved values at first order and for WENO
+        // (the MUSCL face states form their conserved values from the reconstructed primitives).
+        if (locL) {
+            for (int q = 0; q < 5; q++) SL.W[q] = sW[q * T + lL];
+            if constexpr (ORDER != 2)
+                for (int q = 0; q < 4; q++) SL.U[q] = sU[q * T + lL];
         } else {
-            ghost_state(bc, SL, nx, ny, fsv, SR);
+            load_state(Us, f.L, SL);
         }
-    } else {
-        lR = f.R - c0;
-        locR = (unsigned)lR < (unsigned)nct;
-        if (locR) {
+        if (boundary) {
+            // ghost of the cell-centre state (at second order only its primitives are used: the
+            // L side's reconstruction differences toward it)
+            if (bc == BC_EXIT && Uexit) {
+                FState src;
+                load_state(Uexit, f.L, src);
+                ghost_state(bc, src, nx, ny, fsv, SR);
+            } else {
+                ghost_state(bc, SL, nx, ny, fsv, SR);
+            }
+        } else if (locR) {
             for (int q = 0; q < 5; q++) SR.W[q] = sW[q * T + lR];
             if constexpr (ORDER != 2)
                 for (int q = 0; q < 4; q++) SR.U[q] = sU[q * T + lR];
@@ -270,97 +328,56 @@ __device__ __forceinline__ void flux_face(const DevMesh &m, const DevCfg &cfg,
         nb[3 * FT + j] = (float)(boundary ? SL.W[3] : SR.W[3]);
     }
     double F[4];
-    if constexpr (ORDER == 3) {
-        // WENO5 on the conserved variables along the line of quadrilaterals through the face,
-        // cells L-2, L-1, L | R, R+1, R+2, where the layout found one; MUSCL below otherwise
-        const int4 q4 = boundary ? make_int4(-1, -1, -1, -1) : m.fst[e];
-        if (q4.x >= 0) {
-            auto cons = [&](int c, double *u) {
-                const int l = c - c0;
-                if ((unsigned)l < (unsigned)nct) {
-                    for (int q = 0; q < 4; q++) u[q] = sU[q * T + l];
-                } else {
-                    const double4 v = Us[c];
-                    u[0] = v.x;
-                    u[1] = v.y;
-                    u[2] = v.z;
-                    u[3] = v.w;
-                }
-            };
-            double Lm2[4], Lm1[4], Rp1[4], Rp2[4];
-            cons(q4.y, Lm2);
-            cons(q4.x, Lm1);
-            cons(q4.z, Rp1);
-            cons(q4.w, Rp2);
-            double UL[4], UR[4];
-            for (int q = 0; q < 4; q++) {
-                UL[q] = weno5(Lm2[q], Lm1[q], SL.U[q], SR.U[q], Rp1[q], 0);
-                UR[q] = weno5(Lm1[q], SL.U[q], SR.U[q], Rp1[q], Rp2[q], 1);
+    if constexpr (ORDER >= 2) {
+        double gL[8], gR[8];
+        if (!line || VISC) {
+            if (glds && locL) {
+                for (int q = 0; q < 8; q++) gL[q] = sG[q * T + lL];
+            } else {
+                load_grad(grad, f.L, gL);
             }
-            FState fL, fR;
-            weno_face_state(UL, SL, fL);
-            weno_face_state(UR, SR, fR);
-            face_flux<FLUX>(false, cfg.roe_bdiss, fL, fR, nx, ny, dl, F);
+        }
+        if (line) {
             if constexpr (VISC) {
-                double gL[8], gR[8];
-                if (glds && locL) {
-                    for (int q = 0; q < 8; q++) gL[q] = sG[q * T + lL];
-                } else {
-                    load_grad(grad, f.L, gL);
-                }
                 if (glds && locR) {
                     for (int q = 0; q < 8; q++) gR[q] = sG[q * T + lR];
                 } else {
                     load_grad(grad, f.R, gR);
                 }
-                double Fv[4];
-                viscous_flux(cfg, SL.W, SR.W, gL, gR, nx, ny, dl, f.dx, f.dy, Fv);
-                for (int q = 0; q < 4; q++) F[q] = F[q] - Fv[q];
             }
-            for (int q = 0; q < 4; q++) sF[q * FT + j] = F[q];
-            return;
-        }
-    }
-    if constexpr (ORDER >= 2) {
-        double gL[8];
-        if (glds && locL) {
-            for (int q = 0; q < 8; q++) gL[q] = sG[q * T + lL];
         } else {
-            load_grad(grad, f.L, gL);
-        }
-        double gR[8];
-        FState fL, fR;
-        // frozen limiter factors of this face entry: side L in pv[0..3], side R in pv[4..7]
-        // (8 contiguous floats per entry, two 16-byte loads)
-        float pv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        float4 *p4 = fz ? reinterpret_cast<float4 *>(psi) + 2 * (size_t)e : nullptr;
-        if (fz == 2) {
-            const float4 a = p4[0], b = p4[1];
-            pv[0] = a.x; pv[1] = a.y; pv[2] = a.z; pv[3] = a.w;
-            pv[4] = b.x; pv[5] = b.y; pv[6] = b.z; pv[7] = b.w;
-        }
-        reconstruct_side<LIM>(SL, SR, gL, f.dx, f.dy, 1.0, fz, pv, fL);
-        if (boundary) {
-            if (bc == BC_EXIT && Uexit) {
-                FState src;
-                load_state(Uexit, f.L, src);
-                ghost_state(bc, src, nx, ny, fsv, fR);
-            } else {
-                ghost_state(bc, fL, nx, ny, fsv, fR);
+            // frozen limiter factors of this face entry: side L in pv[0..3], side R in pv[4..7]
+            // (8 contiguous floats per entry, two 16-byte loads)
+            float pv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            float4 *p4 = fz ? reinterpret_cast<float4 *>(psi) + 2 * (size_t)e : nullptr;
+            if (fz == 2) {
+                const float4 a = p4[0], b = p4[1];
+                pv[0] = a.x; pv[1] = a.y; pv[2] = a.z; pv[3] = a.w;
+                pv[4] = b.x; pv[5] = b.y; pv[6] = b.z; pv[7] = b.w;
             }
-            if constexpr (VISC)
-                for (int q = 0; q < 8; q++) gR[q] = gL[q];
-        } else {
-            if (glds && locR) {
-                for (int q = 0; q < 8; q++) gR[q] = sG[q * T + lR];
+            reconstruct_side<LIM>(SL, SR, gL, f.dx, f.dy, 1.0, fz, pv, fL);
+            if (boundary) {
+                if (bc == BC_EXIT && Uexit) {
+                    FState src;
+                    load_state(Uexit, f.L, src);
+                    ghost_state(bc, src, nx, ny, fsv, fR);
+                } else {
+                    ghost_state(bc, fL, nx, ny, fsv, fR);
+                }
+                if constexpr (VISC)
+                    for (int q = 0; q < 8; q++) gR[q] = gL[q];
             } else {
-                load_grad(grad, f.R, gR);
+                if (glds && locR) {
+                    for (int q = 0; q < 8; q++) gR[q] = sG[q * T + lR];
+                } else {
+                    load_grad(grad, f.R, gR);
+                }
+                reconstruct_side<LIM>(SR, SL, gR, f.dx, f.dy, -1.0, fz, pv + 4, fR);
             }
-            reconstruct_side<LIM>(SR, SL, gR, f.dx, f.dy, -1.0, fz, pv + 4, fR);
-        }
-        if (fz == 1) {
-            p4[0] = make_float4(pv[0], pv[1], pv[2], pv[3]);
-            p4[1] = make_float4(pv[4], pv[5], pv[6], pv[7]);
+            if (fz == 1) {
+                p4[0] = make_float4(pv[0], pv[1], pv[2], pv[3]);
+                p4[1] = make_float4(pv[4], pv[5], pv[6], pv[7]);
+            }
         }
         face_flux<FLUX>(boundary, cfg.roe_bdiss, fL, fR, nx, ny, dl, F);
         if constexpr (VISC) {
@@ -506,8 +523,9 @@ __global__ void __launch_bounds__(256) CFD_FLUX_ATTR CFD_POS_ATTR flux_tile_kern
         u4 = Us[c];
         if (CFD_FLUX_PREFETCH_CELL) load_cell_inputs();
     }
+    // two faces ahead; at order 3 one copy of the (long) face code runs them all
     FaceRec f0{}, f1{};
-    const bool h0 = k < nft, h1 = k + B < nft;
+    const bool h0 = k < nft && ORDER < 3, h1 = k + B < nft && ORDER < 3;
     if (h0) load_face<true, ORDER >= 2>(m, fs + k, f0);
     if (h1) load_face<true, ORDER >= 2>(m, fs + k + B, f1);
 
@@ -535,7 +553,7 @@ __global__ void __launch_bounds__(256) CFD_FLUX_ATTR CFD_POS_ATTR flux_tile_kern
         stageN(k + B, f1);
         flux_face<FLUX, ORDER, LIM, VISC, POS>(m, cfg, Us, grad, Uexit, sW, sU, sG, sF, glds, T, FT, c0, nct, k + B, f1, fz, st.psi, fs + k + B, fsv, st.pflag, sNb);
     }
-    for (int j = k + 2 * B; j < nft; j += B) {
+    for (int j = k + (ORDER < 3 ? 2 * B : 0); j < nft; j += B) {
         FaceRec f;
         load_face<true, ORDER >= 2>(m, fs + j, f);
         stageN(j, f);
