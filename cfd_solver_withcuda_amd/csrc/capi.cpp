@@ -74,6 +74,47 @@ void capi_fill_viscous(DevCfg &d, const cfd_config_t &c) {
     d.kfac = c.viscous ? 1.4 * c.r_gas / ((1.4 - 1.0) * c.prandtl) : 0.0;
     d.inv_pr = c.viscous ? 1.0 / c.prandtl : 0.0;
 }
+
+HostRows::~HostRows() {
+    if (buf_) (void)hipFree(buf_);
+    if (d_iperm_) (void)hipFree(d_iperm_);
+}
+
+hipError_t HostRows::get(const std::vector<int> &iperm, int w, const double *d, double *h, hipStream_t st) {
+    const size_t n = iperm.size(), need = n * w;
+    if (n == 0) return hipSuccess;
+    std::lock_guard<std::mutex> lock(lock_);
+    hipError_t e = hipSuccess;
+    if (!d_iperm_) {
+        int *p = nullptr;
+        if ((e = hipMalloc((void **)&p, n * sizeof(int))) == hipSuccess &&
+            (e = hipMemcpy(p, iperm.data(), n * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess) {
+            (void)hipFree(p);
+            return e;
+        }
+        d_iperm_ = p;
+    }
+    if (e == hipSuccess && need > cap_) {
+        if (buf_) (void)hipFree(buf_);
+        buf_ = nullptr;
+        cap_ = 0;
+        if ((e = hipMalloc((void **)&buf_, need * sizeof(double))) == hipSuccess) cap_ = need;
+    }
+    if (e == hipSuccess) {
+        if ((e = launch_order_rows(d_iperm_, n, w, d, buf_, st)) != hipSuccess ||
+            (e = hipMemcpyAsync(h, buf_, need * sizeof(double), hipMemcpyDeviceToHost, st)) != hipSuccess)
+            return e;
+        return hipStreamSynchronize(st);
+    }
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();  // no room: ordered by the host
+    std::vector<double> t(need);
+    if ((e = hipMemcpyAsync(t.data(), d, need * sizeof(double), hipMemcpyDeviceToHost, st)) != hipSuccess ||
+        (e = hipStreamSynchronize(st)) != hipSuccess)
+        return e;
+    for (size_t c = 0; c < n; c++) std::memcpy(&h[c * w], &t[(size_t)iperm[c] * w], w * sizeof(double));
+    return hipSuccess;
+}
 }  // namespace cfd
 
 struct cfd_solver_s {
@@ -102,6 +143,7 @@ struct cfd_solver_s {
     int cur = 0;
     bool dt_valid = false;
     bool has_state = false;
+    HostRows rows;
     ~cfd_solver_s() {
         void *ps[] = {Un, Ua, Ub, acc, R, dt, grad, hbuf, err_partial, dt_partial, scal, Ug, psi, fz, fz_best, Uall,
                       Uc, acc2, pflag, dirty};
@@ -462,11 +504,8 @@ int cfd_set_state(cfd_solver_t *s, const double *U) {
 
 int cfd_get_state(cfd_solver_t *s, double *U) {
     if (!s || !U) return fail(CFD_E_ARG, "cfd_get_state: null argument");
-    const int nc = s->m->ref.nc;
-    std::vector<double> h(4 * (size_t)nc);
     HIP_TRY(hipDeviceSynchronize());
-    HIP_TRY(hipMemcpy(h.data(), s->Un, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-    for (int k = 0; k < nc; k++) std::memcpy(&U[4 * (size_t)s->m->lay.perm[k]], &h[4 * (size_t)k], 4 * sizeof(double));
+    HIP_TRY(s->rows.get(s->m->lay.iperm, 4, reinterpret_cast<const double *>(s->Un), U, nullptr));
     return 0;
 }
 
@@ -566,24 +605,12 @@ int cfd_residual(cfd_solver_t *s, double *R, double *dt, double *grad, void *str
     hipStream_t st = (hipStream_t)stream;
     int rc = residual_pass(s, s->Un, nullptr, nullptr, st, 0, grad != nullptr);
     if (rc) return rc;
+    const std::vector<int> &iperm = s->m->lay.iperm;
+    // the widest first, which sizes the ordered rows
+    if (grad && s->cfg.order >= 2) HIP_TRY(s->rows.get(iperm, 8, s->grad, grad, st));
+    if (R) HIP_TRY(s->rows.get(iperm, 4, reinterpret_cast<const double *>(s->R), R, st));
+    if (dt) HIP_TRY(s->rows.get(iperm, 1, s->dt, dt, st));
     HIP_TRY(hipStreamSynchronize(st));
-    const int nc = s->m->ref.nc;
-    const std::vector<int> &perm = s->m->lay.perm;
-    if (R) {
-        std::vector<double> h(4 * (size_t)nc);
-        HIP_TRY(hipMemcpy(h.data(), s->R, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-        for (int k = 0; k < nc; k++) std::memcpy(&R[4 * (size_t)perm[k]], &h[4 * (size_t)k], 4 * sizeof(double));
-    }
-    if (dt) {
-        std::vector<double> h(nc);
-        HIP_TRY(hipMemcpy(h.data(), s->dt, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-        for (int k = 0; k < nc; k++) dt[perm[k]] = h[k];
-    }
-    if (grad && s->cfg.order >= 2) {
-        std::vector<double> h(8 * (size_t)nc);
-        HIP_TRY(hipMemcpy(h.data(), s->grad, h.size() * sizeof(double), hipMemcpyDeviceToHost));
-        for (int k = 0; k < nc; k++) std::memcpy(&grad[8 * (size_t)perm[k]], &h[8 * (size_t)k], 8 * sizeof(double));
-    }
     return 0;
 }
 

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "fv_kernels.h"
+#include "host_rows.h"
 #include "mesh_host.h"
 
 using namespace cfd;
@@ -109,6 +110,7 @@ struct cfd_batch_s {
     cfd_progress_fn progress = nullptr;  // called every progress_every checks of a solve
     void *progress_user = nullptr;
     int progress_every = 0;
+    HostRows rows;
     double build_s = 0.0, tune_s = 0.0;
     int tune_src = 0;  // launch shape: 0 given, 1 timed by the autotuner, 2 from the autotune cache
     ~cfd_batch_s() {
@@ -798,16 +800,7 @@ int cfd_batch_set_state(cfd_batch_t *b, const double *U) {
 
 int cfd_batch_get_state(cfd_batch_t *b, double *U) {
     if (!b || !U) return capi_fail(CFD_E_ARG, "cfd_batch_get_state: null argument");
-    std::vector<double4> h(b->nc);
-    BHIP(hipStreamSynchronize(b->stream));
-    BHIP(hipMemcpy(h.data(), b->Un, h.size() * sizeof(double4), hipMemcpyDeviceToHost));
-    for (int c = 0; c < b->nc; c++) {
-        const double4 q = h[b->iperm[c]];
-        U[4 * (size_t)c] = q.x;
-        U[4 * (size_t)c + 1] = q.y;
-        U[4 * (size_t)c + 2] = q.z;
-        U[4 * (size_t)c + 3] = q.w;
-    }
+    BHIP(b->rows.get(b->iperm, 4, reinterpret_cast<const double *>(b->Un), U, b->stream));
     return 0;
 }
 

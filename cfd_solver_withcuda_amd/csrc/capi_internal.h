@@ -7,6 +7,7 @@
 
 #include "../../include/cfd_hip.h"
 #include "cfd_types.h"
+#include "host_rows.h"
 #include "mesh_host.h"
 
 using cfd::DevMesh;

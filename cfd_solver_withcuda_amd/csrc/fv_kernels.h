@@ -81,6 +81,9 @@ hipError_t launch_flux_weno_visc(const DevMesh &m, const DevCfg &c, int flux, in
                                  size_t sm, hipStream_t s);
 hipError_t launch_fill(double *p, double v, int n, hipStream_t s);
 hipError_t launch_err_finalize(const double *partial, int n, double *err4, hipStream_t s);
+// out[c w + q] = in[iperm[c] w + q], c < n, q < w (1, 4 or 8).
+hipError_t launch_order_rows(const int *iperm, size_t n, int w, const double *in, double *out, hipStream_t s);
+
 hipError_t launch_ghosts(int n, const int *gcell, const double2 *gnrm, const int *gkind,
                          const DevCfg &c, const double4 *Us, const double4 *Uexit, double4 *Ug,
                          hipStream_t s);

@@ -211,6 +211,15 @@ __global__ void __launch_bounds__(1024) err_finalize_kernel(const double *partia
         for (int q = 0; q < 4; q++) err4[q] = sqrt(red[q * B]);
 }
 
+// Rows of W doubles in the caller's cell order, one value per thread: the writes are contiguous, the
+// reads whole rows of a tile's neighbourhood.
+template <int W>
+__global__ void __launch_bounds__(256) order_rows_kernel(const int *__restrict__ iperm, size_t n,
+                                                         const double *__restrict__ in, double *__restrict__ out) {
+    const size_t e = blockIdx.x * (size_t)256 + threadIdx.x;
+    if (e < n * W) out[e] = in[(size_t)iperm[e / W] * W + e % W];
+}
+
 // Ghost states of the boundary faces (Apply_Boundary_Conditions, src/Boundary_Conditions.cpp:12-61):
 // ghost k of owner cell gcell[k] across a face of kind gkind[k] with unit normal gnrm[k].
 __global__ void __launch_bounds__(256) ghost_kernel(int n, const int *__restrict__ gcell,
@@ -761,6 +770,15 @@ hipError_t launch_roe2o(int nc, const RefCells &rc, const double4 *U_all, double
                         double cfl, double4 *R, double *dt, double *dt_partial, hipStream_t s) {
     if (nc <= 0) return hipSuccess;
     hipLaunchKernelGGL(roe2o_kernel, dim3((nc + 255) / 256), dim3(256), 0, s, nc, rc, U_all, zeta, zeta1, cfl, R, dt, dt_partial);
+    return hipGetLastError();
+}
+
+hipError_t launch_order_rows(const int *iperm, size_t n, int w, const double *in, double *out, hipStream_t s) {
+    const dim3 grid((unsigned)((n * w + 255) / 256));
+    if (w == 1) hipLaunchKernelGGL(order_rows_kernel<1>, grid, dim3(256), 0, s, iperm, n, in, out);
+    else if (w == 4) hipLaunchKernelGGL(order_rows_kernel<4>, grid, dim3(256), 0, s, iperm, n, in, out);
+    else if (w == 8) hipLaunchKernelGGL(order_rows_kernel<8>, grid, dim3(256), 0, s, iperm, n, in, out);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
