@@ -84,7 +84,7 @@ struct cfd_batch_s {
     int *d_rings = nullptr, *d_ring_cell = nullptr, *d_ghost = nullptr;
     uint16_t *d_own_nbr = nullptr, *d_ring_nbr = nullptr, *d_floc = nullptr;
     int *d_tile_inst = nullptr, *d_inst_tile = nullptr, *d_tile_list = nullptr, *d_tile_count = nullptr;
-    int *d_inst_off = nullptr, *d_status = nullptr, *d_steps = nullptr;
+    int *d_status = nullptr, *d_steps = nullptr;
     int *d_fz = nullptr, *d_fz_since = nullptr;  // per instance limiter-freezing state
     double *d_fz_best = nullptr;
     float *psi = nullptr;  // [8 * face entries] frozen limiter factors
@@ -100,8 +100,8 @@ struct cfd_batch_s {
     double *grad = nullptr, *hbuf = nullptr, *err_partial = nullptr;
     DevMesh dev{};
     hipStream_t stream = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    hipGraph_t graph = nullptr, graph_many = nullptr;
+    hipGraphExec_t exec = nullptr, exec_many = nullptr;  // one step, kGraphSteps steps
     double graph_tol = -1.0;
     int graph_tiles = 0;         // tiles the captured step's launch grids cover
     std::vector<int> fz_start;   // per instance freeze mode each solve starts with (empty: 0)
@@ -114,11 +114,13 @@ struct cfd_batch_s {
     double build_s = 0.0, tune_s = 0.0;
     int tune_src = 0;  // launch shape: 0 given, 1 timed by the autotuner, 2 from the autotune cache
     ~cfd_batch_s() {
-        if (exec) (void)hipGraphExecDestroy(exec);
-        if (graph) (void)hipGraphDestroy(graph);
+        for (hipGraphExec_t e : {exec, exec_many})
+            if (e) (void)hipGraphExecDestroy(e);
+        for (hipGraph_t g : {graph, graph_many})
+            if (g) (void)hipGraphDestroy(g);
         if (stream) (void)hipStreamDestroy(stream);
         void *ps[] = {d_tile_cstart, d_tile_fstart, d_fgeo, d_cw, d_cn, d_ghost_n, d_fd, d_rings, d_ring_cell, d_ghost, d_own_nbr, d_ring_nbr, d_floc, d_fnx, d_fny, d_fdl, d_fLR, d_fst, d_area, d_inv_area, d_slots, d_tile_inst, d_inst_tile,
-                      d_tile_list, d_tile_count, d_inst_off, d_status, d_steps, d_inst_fs, d_err4,
+                      d_tile_list, d_tile_count, d_status, d_steps, d_inst_fs, d_err4,
                       Un, Ua, Ub, acc, grad, hbuf, err_partial, d_fz, d_fz_since, d_fz_best, psi,
                       Uc, acc2, pflag, dirty};
         for (void *p : ps)
@@ -271,7 +273,6 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
     BALLOC(b->d_inst_tile, (size_t)ni + 1);
     BALLOC(b->d_tile_list, nt);
     BALLOC(b->d_tile_count, 1);
-    BALLOC(b->d_inst_off, (size_t)ni);
     BALLOC(b->d_status, (size_t)ni);
     BALLOC(b->d_steps, (size_t)ni);
     BALLOC(b->d_inst_fs, (size_t)ni);
@@ -435,8 +436,8 @@ int batch_reset(cfd_batch_s *b) {
         BHIP(h2d(b->d_fz_since, zeros.data(), zeros.size()));
         BHIP(h2d(b->d_fz_best, big.data(), big.size()));
     }
-    BHIP(launch_batch_list(b->ninst, b->ntiles, b->d_inst_tile, b->d_tile_inst, b->d_status,
-                           b->d_inst_off, b->d_tile_list, b->d_tile_count, b->stream));
+    BHIP(launch_batch_list(b->ninst, b->ntiles, b->d_inst_tile, b->d_tile_inst, b->d_status, b->d_tile_list,
+                           b->d_tile_count, b->stream));
     return 0;
 }
 
@@ -495,35 +496,54 @@ int batch_step_launches(cfd_batch_s *b, double tol, int grid_tiles) {
     if (pos) BHIP(launch_batch_commit(dm, grid_tiles, b->Uc, b->Un, b->stream));
     BHIP(launch_batch_status(b->ninst, b->d_inst_tile, b->err_partial, tol, b->d_status, b->d_steps, b->d_err4,
                              b->d_fz, b->d_fz_best, b->d_fz_since, c.freeze_tol, c.freeze_stall, b->stream));
-    BHIP(launch_batch_list(b->ninst, b->ntiles, b->d_inst_tile, b->d_tile_inst, b->d_status,
-                           b->d_inst_off, b->d_tile_list, b->d_tile_count, b->stream));
+    BHIP(launch_batch_list(b->ninst, b->ntiles, b->d_inst_tile, b->d_tile_inst, b->d_status, b->d_tile_list,
+                           b->d_tile_count, b->stream));
+    return 0;
+}
+
+// Captures `steps` steps into *g and *exec (replacing what they held).
+int batch_capture(cfd_batch_s *b, double tol, int grid_tiles, int steps, hipGraph_t *g, hipGraphExec_t *exec) {
+    if (*exec) BHIP(hipGraphExecDestroy(*exec));
+    *exec = nullptr;
+    if (*g) BHIP(hipGraphDestroy(*g));
+    *g = nullptr;
+    BHIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+    int rc = 0;
+    for (int k = 0; k < steps && !rc; k++) rc = batch_step_launches(b, tol, grid_tiles);
+    hipGraph_t got = nullptr;
+    hipError_t e = hipStreamEndCapture(b->stream, &got);
+    if (rc) {
+        if (got) (void)hipGraphDestroy(got);
+        return rc;
+    }
+    if (e != hipSuccess) return capi_hip_fail(e, "hipStreamEndCapture");
+    *g = got;
+    BHIP(hipGraphInstantiate(exec, *g, nullptr, nullptr, 0));
     return 0;
 }
 
 int batch_graph(cfd_batch_s *b, double tol, int grid_tiles = -1) {
     if (grid_tiles < 0) grid_tiles = b->ntiles;
     if (b->exec && b->graph_tol == tol && b->graph_tiles == grid_tiles) return 0;
-    if (b->exec) {
-        BHIP(hipGraphExecDestroy(b->exec));
-        b->exec = nullptr;
-    }
-    if (b->graph) {
-        BHIP(hipGraphDestroy(b->graph));
-        b->graph = nullptr;
-    }
-    BHIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    int rc = batch_step_launches(b, tol, grid_tiles);
-    hipGraph_t g = nullptr;
-    hipError_t e = hipStreamEndCapture(b->stream, &g);
-    if (rc) {
-        if (g) (void)hipGraphDestroy(g);
-        return rc;
-    }
-    if (e != hipSuccess) return capi_hip_fail(e, "hipStreamEndCapture");
-    b->graph = g;
-    BHIP(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
+    if (b->exec_many) BHIP(hipGraphExecDestroy(b->exec_many));
+    b->exec_many = nullptr;
+    if (int rc = batch_capture(b, tol, grid_tiles, 1, &b->graph, &b->exec)) return rc;
     b->graph_tol = tol;
     b->graph_tiles = grid_tiles;
+    return 0;
+}
+
+// `n` steps of the captured kind. The device idles 9 us between two graphs, so longer runs replay
+// graphs of several steps (captured when a run first has kMany of them).
+constexpr int kGraphSteps = 8, kMany = 2 * kGraphSteps;
+int batch_many(cfd_batch_s *b, int n) {
+    if (n < kMany || b->exec_many) return 0;
+    return batch_capture(b, b->graph_tol, b->graph_tiles, kGraphSteps, &b->graph_many, &b->exec_many);
+}
+int batch_launch(cfd_batch_s *b, int n) {
+    if (int rc = batch_many(b, n)) return rc;
+    for (; n >= kGraphSteps && b->exec_many; n -= kGraphSteps) BHIP(hipGraphLaunch(b->exec_many, b->stream));
+    for (; n > 0; n--) BHIP(hipGraphLaunch(b->exec, b->stream));
     return 0;
 }
 
@@ -533,12 +553,12 @@ int batch_time_steps(cfd_batch_s *b, int n, double *ms) {
     if (rc) return rc;
     rc = batch_graph(b, -1.0);  // tol < 0: nothing converges while timing
     if (rc) return rc;
-    BHIP(hipGraphLaunch(b->exec, b->stream));
+    if ((rc = batch_many(b, n)) || (rc = batch_launch(b, 1))) return rc;
     hipEvent_t e0, e1;
     BHIP(hipEventCreate(&e0));
     BHIP(hipEventCreate(&e1));
     BHIP(hipEventRecord(e0, b->stream));
-    for (int k = 0; k < n; k++) BHIP(hipGraphLaunch(b->exec, b->stream));
+    if ((rc = batch_launch(b, n))) return rc;
     BHIP(hipEventRecord(e1, b->stream));
     BHIP(hipEventSynchronize(e1));
     float f = 0.f;
@@ -558,7 +578,7 @@ int batch_march(cfd_batch_s *b, int n) {
     if (rc) return rc;
     rc = batch_graph(b, -1.0);
     if (rc) return rc;
-    for (int k = 0; k < n; k++) BHIP(hipGraphLaunch(b->exec, b->stream));
+    if ((rc = batch_launch(b, n))) return rc;
     BHIP(hipStreamSynchronize(b->stream));
     return 0;
 }
@@ -824,7 +844,7 @@ int cfd_batch_solve(cfd_batch_t *b, double tol, int max_steps, int check_every, 
     b->hist_checks = 0;
     while (done < max_steps && !all) {
         const int k = std::min(check_every, max_steps - done);
-        for (int j = 0; j < k; j++) BHIP(hipGraphLaunch(b->exec, b->stream));
+        if ((rc = batch_launch(b, k))) return rc;
         done += k;
         BHIP(hipMemcpyAsync(st.data(), b->d_status, ni * sizeof(int), hipMemcpyDeviceToHost, b->stream));
         BHIP(hipMemcpyAsync(e4.data(), b->d_err4, e4.size() * sizeof(double), hipMemcpyDeviceToHost, b->stream));

@@ -94,8 +94,7 @@ hipError_t launch_batch_status(int ninst, const int *inst_tile, const double *er
 // bounds the marching count.
 hipError_t launch_batch_commit(const DevMesh &m, int grid_tiles, const double4 *src, double4 *dst, hipStream_t s);
 hipError_t launch_batch_list(int ninst, int ntiles, const int *inst_tile, const int *tile_inst,
-                             const int *status, int *inst_off, int *tile_list, int *tile_count,
-                             hipStream_t s);
+                             const int *status, int *tile_list, int *tile_count, hipStream_t s);
 // Freezing state machine of one solve after a step whose error norm is err4[0] (see
 // fv_kernels.hip, freeze_update_kernel).
 hipError_t launch_freeze_update(const double *err4, int *freeze, double *best, int *since,

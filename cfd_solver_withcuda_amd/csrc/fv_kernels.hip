@@ -450,44 +450,52 @@ __global__ void __launch_bounds__(256) batch_status_kernel(const int *__restrict
     }
 }
 
-// Offsets of the marching instances' tiles in the compacted tile list, and its length. One
-// workgroup of 1024 threads scans the instances in chunks of 1024.
-__global__ void __launch_bounds__(1024) batch_list_scan_kernel(int ninst, const int *__restrict__ inst_tile,
-                                                               const int *__restrict__ status,
-                                                               int *__restrict__ inst_off,
-                                                               int *__restrict__ tile_count) {
-    __shared__ int buf[1024];
-    const int t = threadIdx.x;
-    int carry = 0;
-    for (int base = 0; base < ninst; base += 1024) {
-        const int i = base + t;
-        const int v = (i < ninst && status[i] == 1) ? inst_tile[i + 1] - inst_tile[i] : 0;
-        buf[t] = v;
-        __syncthreads();
-        for (int d = 1; d < 1024; d <<= 1) {
-            const int add = (t >= d) ? buf[t - d] : 0;
-            __syncthreads();
-            buf[t] += add;
-            __syncthreads();
-        }
-        if (i < ninst) inst_off[i] = carry + buf[t] - v;
-        carry += buf[1023];
+// The compacted list of the marching instances' tiles, in order, and its length. A workgroup places 256
+// tiles: it counts the marching tiles of the instances before its first one, and scans the 256
+// instances from there on (its tiles' instances, none of which is empty) in LDS. With the scan a
+// launch of its own a step took 5 us and a launch more.
+__global__ void __launch_bounds__(256) batch_list_kernel(int ninst, int ntiles, const int *__restrict__ tile_inst,
+                                                         const int *__restrict__ inst_tile,
+                                                         const int *__restrict__ status, int *__restrict__ tile_list,
+                                                         int *__restrict__ tile_count) {
+    __shared__ int buf[256], sum[256];
+    const int t = threadIdx.x, j = blockIdx.x * 256 + t;
+    const int i0 = tile_inst[blockIdx.x * 256];
+    auto marching = [&](int i) { return status[i] == 1 ? inst_tile[i + 1] - inst_tile[i] : 0; };
+    const int v = i0 + t < ninst ? marching(i0 + t) : 0;
+    int before = 0, after = 0;
+    for (int i = t; i < i0; i += 256) before += marching(i);
+    if (blockIdx.x == 0)
+        for (int i = i0 + 256 + t; i < ninst; i += 256) after += marching(i);
+    buf[t] = v;
+    sum[t] = before;
+    __syncthreads();
+    for (int d = 128; d > 0; d >>= 1) {
+        if (t < d) sum[t] += sum[t + d];
         __syncthreads();
     }
-    if (t == 0) *tile_count = carry;
-}
-
-// Writes the compacted list: tile j of marching instance i goes to inst_off[i] + j - inst_tile[i].
-__global__ void __launch_bounds__(256) batch_list_fill_kernel(int ntiles, const int *__restrict__ tile_inst,
-                                                              const int *__restrict__ inst_tile,
-                                                              const int *__restrict__ status,
-                                                              const int *__restrict__ inst_off,
-                                                              int *__restrict__ tile_list) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= ntiles) return;
-    const int i = tile_inst[j];
-    if (status[i] != 1) return;
-    tile_list[inst_off[i] + j - inst_tile[i]] = j;
+    for (int d = 1; d < 256; d <<= 1) {
+        const int add = t >= d ? buf[t - d] : 0;
+        __syncthreads();
+        buf[t] += add;
+        __syncthreads();
+    }
+    const int base = sum[0];
+    if (j < ntiles) {
+        const int i = tile_inst[j], n = marching(i);
+        if (n) tile_list[base + buf[i - i0] - n + j - inst_tile[i]] = j;
+    }
+    if (blockIdx.x == 0) {  // i0 = 0 here: nothing before
+        const int first = buf[255];
+        __syncthreads();
+        sum[t] = after;
+        __syncthreads();
+        for (int d = 128; d > 0; d >>= 1) {
+            if (t < d) sum[t] += sum[t + d];
+            __syncthreads();
+        }
+        if (t == 0) *tile_count = first + sum[0];
+    }
 }
 
 // Minimum of n per-tile partial minima (fmin ignores NaN, as the reference's `<` scan does).
@@ -757,12 +765,10 @@ hipError_t launch_batch_commit(const DevMesh &m, int grid_tiles, const double4 *
 }
 
 hipError_t launch_batch_list(int ninst, int ntiles, const int *inst_tile, const int *tile_inst,
-                             const int *status, int *inst_off, int *tile_list, int *tile_count,
-                             hipStream_t s) {
-    hipLaunchKernelGGL(batch_list_scan_kernel, dim3(1), dim3(1024), 0, s, ninst, inst_tile, status, inst_off, tile_count);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || ntiles <= 0) return e;
-    hipLaunchKernelGGL(batch_list_fill_kernel, dim3((ntiles + 255) / 256), dim3(256), 0, s, ntiles, tile_inst, inst_tile, status, inst_off, tile_list);
+                             const int *status, int *tile_list, int *tile_count, hipStream_t s) {
+    if (ntiles <= 0) return hipErrorInvalidValue;  // every instance has a cell
+    hipLaunchKernelGGL(batch_list_kernel, dim3((ntiles + 255) / 256), dim3(256), 0, s, ninst, ntiles, tile_inst, inst_tile,
+                       status, tile_list, tile_count);
     return hipGetLastError();
 }
 
