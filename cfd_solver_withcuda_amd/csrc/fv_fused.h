@@ -490,8 +490,8 @@ __global__ void __launch_bounds__(VISC || POS == 2 ? 512 : 1024) fused_tile_kern
             }
             const double Un[4] = {un4.x, un4.y, un4.z, un4.w};
             const double us[4] = {us4.x, us4.y, us4.z, us4.w};
-            double Uo[4];
-            stage_update(st, c, h, Un, us, us4, r, Uo);
+            const double4 o4 = stage_update(st, c, h, Un, us, us4, r);
+            const double Uo[4] = {o4.x, o4.y, o4.z, o4.w};
             if constexpr (POS == 1) {
                 // positivity fallback, detection (the same test as flux_tile_kernel's): the range of
                 // the cell's and its face neighbours' stage inputs, rounded to FP32
@@ -511,7 +511,7 @@ __global__ void __launch_bounds__(VISC || POS == 2 ? 512 : 1024) fused_tile_kern
                 st.pflag[c] = bad ? 1 : 0;
                 if (bad) mark_dirty(m, st, tile, c0, nct, fs, sls);
             }
-            st.Uout[c] = make_double4(Uo[0], Uo[1], Uo[2], Uo[3]);
+            st.Uout[c] = o4;
             if (st.last) {
                 if (st.err_partial) {
                     for (int q = 0; q < 4; q++) errp[q] += err_term(Uo[q] - Un[q], Un[q]);
