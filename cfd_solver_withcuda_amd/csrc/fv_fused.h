@@ -10,10 +10,11 @@
 // of 128 Hilbert-ordered cells, each at about a sixth of a face flux's arithmetic), which costs less
 // than the traffic. Measured on MI355X, whole steps, two-pass to one launch: 7.97M-cell forward
 // step, RK4 with the positivity fallback 3.83 to 2.80 ms; 1.27M-cell bump, RK3 0.423 to 0.332 ms;
-// 320k-cell viscous bump 161 to 118 us; 2.5k cells 50 to 32 us.
+// 320k-cell viscous bump 161 to 118 us; 2.5k cells 50 to 32 us (and with stage_update's states kept
+// in registers to 2.61 ms, 0.307 ms, 113 us and 31 us).
 //
-// What bounds it (forward step, 0.70 ms a stage): FP64 issue, 2,040 vector instructions a wave or
-// 72 % of the launch; the L2 fills run at 4.4 TB/s, 95 % of a large copy's rate on the same card.
+// What bounds it (forward step, 0.65 ms a stage): FP64 issue, about 2,000 vector instructions a wave or
+// 70-75 % of the launch; the L2 fills run at 4.4-4.9 TB/s, the rate of a large copy on the same card.
 // Neither leaves room for less occupancy: 128 registers and 20 KB of LDS give 4 waves per SIMD, and
 // every variant that spilled (a second prefetched stencil for Green-Gauss, initialised records) lost
 // more than it hid.
