@@ -9,6 +9,7 @@ reproduces the CPU restatement's rounding, and with packed FP32 ops disabled.
 """
 from __future__ import annotations
 
+import hashlib
 import os
 import subprocess
 import sys
@@ -38,12 +39,25 @@ def _hipcc() -> str:
     return "hipcc"
 
 
+def kernel_digest(defines: tuple = (), flags: tuple = ()) -> str:
+    """Digest of what decides a batched step's time: the sources of its kernels, launches and tiled
+    layout, and the options they are built with. The autotune cache keeps it in its keys."""
+    h = hashlib.sha1(repr((COMMON[:-1], HIP_FLAGS, defines, flags)).encode())
+    for name in sorted(os.listdir(CSRC)):
+        if name.startswith(("fv_", "cfd_types", "mesh_host", "capi_batch")):
+            with open(os.path.join(CSRC, name), "rb") as f:
+                h.update(name.encode() + b"\0" + f.read())
+    return "k" + h.hexdigest()[:12]
+
+
 def _compile(src: str, build_dir: str = BUILD, defines: tuple = (), flags: tuple = ()) -> str:
     path = os.path.join(CSRC, src)
     obj = os.path.join(build_dir, os.path.splitext(src)[0] + ".o")
     cmd = [_hipcc()] + COMMON + [f"-D{d}" for d in defines]
     if src.endswith(".hip"):
         cmd += HIP_FLAGS + list(flags)
+    if src == "capi_batch.cpp":
+        cmd.append(f"-DCFD_KERNELS={kernel_digest(tuple(defines), tuple(flags))}")
     cmd += ["-c", path, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

@@ -585,9 +585,9 @@ int batch_march(cfd_batch_s *b, int n) {
 
 // ---- autotune cache --------------------------------------------------------------------------
 // One JSON object in a file, one entry per line: "key": [tile, face budget, block, ms per cell].
-// The key names the GPU (architecture, compute units) and the batch's statistics (instances, total
-// and largest cell counts in powers of two) and scheme, so a batch of the same shape on the same
-// GPU reuses the measured choice. Path: CFD_AUTOTUNE_CACHE, else $HOME/.cache/cfdhip_autotune.json;
+// The key names the GPU (architecture, compute units), the batch's statistics (instances, total
+// and largest cell counts in powers of two), the scheme and the kernels, so a batch of the same shape
+// on the same GPU reuses the measured choice. Path: CFD_AUTOTUNE_CACHE, else $HOME/.cache/cfdhip_autotune.json;
 // an unreadable or unwritable file only disables the cache.
 std::string tune_cache_path() {
     if (const char *p = std::getenv("CFD_AUTOTUNE_CACHE")) return p;
@@ -603,6 +603,15 @@ int ilog2(long v) {
     }
     return k;
 }
+
+// The kernels that a cached shape was timed with: the build gives a digest of their sources and flags, so
+// that an entry of other kernels is not found. (The one-launch second-order pass moved the ramps' best
+// shape from 128-cell to 256-cell tiles.)
+#ifndef CFD_KERNELS
+#error "CFD_KERNELS: digest of the kernel sources (build.py)"
+#endif
+#define CFD_TEXT_(x) #x
+#define CFD_TEXT(x) CFD_TEXT_(x)
 
 std::string tune_key(const cfd_config_t &c, const std::vector<InstanceInput> &in) {
     int dev = 0;
@@ -621,7 +630,8 @@ std::string tune_key(const cfd_config_t &c, const std::vector<InstanceInput> &in
     std::ostringstream k;
     k << arch << ":" << cus << "|inst2^" << ilog2((long)in.size()) << "|cells2^" << ilog2(total) << "|max2^"
       << ilog2(largest) << "|order" << c.order << "|flux" << c.flux << "|lim" << c.limiter << "|grad"
-      << c.gradient << "|visc" << c.viscous << "|rk" << c.rk;
+      << c.gradient << "|visc" << c.viscous << "|rk" << c.rk << "|pos" << c.positivity << "|freeze"
+      << (c.freeze_tol > 0.0 || c.freeze_stall > 0) << "|kernels" CFD_TEXT(CFD_KERNELS);
     std::string s = k.str();
     for (char &ch : s)
         if (ch == '"' || ch == '\\') ch = '_';

@@ -205,8 +205,9 @@ int cfd_batch_info(const cfd_batch_t *b, int *out8, double *secs2);
 /* Where the launch shape came from: *source = 0 given (cfg->block), 1 timed by the autotuner
  * (each candidate marched 200 steps from freestream, then 5 timed steps), 2 read from the autotune
  * cache (a JSON file, CFD_AUTOTUNE_CACHE or $HOME/.cache/cfdhip_autotune.json, keyed by the GPU's
- * architecture and compute units and the batch's instance count, total and largest cell counts
- * in powers of two, and scheme). */
+ * architecture and compute units, the batch's instance count, total and largest cell counts
+ * in powers of two, the scheme and a digest of the kernels' sources: another build's entries are
+ * not used). */
 int cfd_batch_tuning(const cfd_batch_t *b, int *source);
 /* U[4*total cells] conserved, instances concatenated in order, each in its caller's cell order */
 int cfd_batch_set_state(cfd_batch_t *b, const double *U);
