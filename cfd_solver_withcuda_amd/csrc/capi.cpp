@@ -264,6 +264,7 @@ int cfd_mesh_create(int npts, const double *pts3, int ncells, const int *cells4,
         d.floc = reinterpret_cast<const ushort2 *>(m->d_floc);
         d.max_local = rings.max_local;
         d.max_grad = rings.max_grad;
+        d.first_ring = rings.first_ring;
     }
     d.fLR = reinterpret_cast<const int2 *>(m->d_fLR);
     d.fnx = m->d_fnx;

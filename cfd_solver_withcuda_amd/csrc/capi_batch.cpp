@@ -235,6 +235,7 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
         gh_off[i + 1] = gh_off[i] + rgs[i].ghost.size() / 2;
         b->dev.max_local = std::max(b->dev.max_local, rgs[i].max_local);
         b->dev.max_grad = std::max(b->dev.max_grad, rgs[i].max_grad);
+        b->dev.first_ring += rgs[i].first_ring;
     }
     rings = rings && rc_off[ni] <= 0x7FFFFFFFu;
     b->nc = b->cell_off[ni];

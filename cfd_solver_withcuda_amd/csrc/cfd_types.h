@@ -62,6 +62,7 @@ struct DevMesh {
     const ushort2 *floc;      // [nfe] local cells of L and R (R: the ghost on a boundary face)
     const double *cn;         // [12*nc] outward unit normal and length per face slot (Green-Gauss; lazily built)
     int max_local, max_grad;  // most local cells, and cells with gradients, of a tile
+    long first_ring;          // first-ring cells of all tiles
     // Batched meshes (several independent instances concatenated; null for one mesh):
     const int *tile_inst;     // [ntiles] instance of each tile
     const double4 *inst_fs;   // [ninst] prescribed state (rho, u, v, p) of each instance

@@ -53,7 +53,7 @@ hipError_t launch_flux_pos(const DevMesh &m, const DevCfg &c, int flux, int lim,
                            const double4 *Us, const double *grad, const StageArgs &st, int block,
                            hipStream_t s);
 // Second-order passes: the residual (R, dt and, when grad_out, the gradients) or one stage with
-// pos = 0, or the positivity fallback's pass pos = 1 or 2. Where the tiles' neighbourhoods fit
+// pos = 0, or the positivity fallback's pass pos = 1 or 2. Where that is the faster form
 // (fused_fits) a pass is one launch (fv_fused.h); otherwise a gradient pass into `grad` comes first
 // (not before pos = 2, which reads pass 1's).
 bool fused_fits(const DevMesh &m, const DevCfg &c, int gradient, int block);

@@ -15,6 +15,7 @@
 #include <algorithm>
 
 #include "fv_fused.h"
+#include "mesh_host.h"
 
 namespace cfd {
 
@@ -675,11 +676,12 @@ hipError_t launch_flux(const DevMesh &m, const DevCfg &c, int flux, int order, i
     return launch_flux_family<2, false>(m, c, flux, lim, mode, Us, grad, st, block, sm, s);
 }
 
-// The one-launch pass runs where its LDS lets at least two workgroups share a compute unit, and
-// not with persistent workgroups (a launch mode of the two-pass kernels).
+// The one-launch pass runs where it is the faster form, and not with persistent workgroups (a launch
+// mode of the two-pass kernels).
 bool fused_fits(const DevMesh &m, const DevCfg &c, int gradient, int block) {
     if (!m.rings || c.persist || (gradient == GRAD_GG && !m.cn)) return false;
-    return sizeof(double) * fused_doubles(m.max_local, m.max_grad, m.max_tile_faces, block, block) <= 65536;
+    const size_t lds = sizeof(double) * fused_doubles(m.max_local, m.max_grad, m.max_tile_faces, block, block);
+    return one_launch_pays(m.nc, m.ntiles, m.first_ring, lds, block);
 }
 
 // Threads of a one-launch pass: the configuration's block, except where the launch leaves compute

@@ -485,8 +485,29 @@ void tile_rings(const RefMesh &m, const Layout &L, TileRings &r) {
         r.tiles.insert(r.tiles.end(), rec, rec + 4);
         r.max_local = std::max(r.max_local, nct + nr + ng);
         r.max_grad = std::max(r.max_grad, nct + n1);
+        r.first_ring += n1;
     }
     r.ok = true;
+}
+
+// Against the two launches (gradients, then fluxes) the one launch saves the gradients' way through
+// memory and a launch, and pays with the ring's gradients and the LDS of the ring's states. Steps on
+// MI355X, two launches over one, 9k to 936k cells, tiles of 16 to 256, cells in Hilbert order, by rows,
+// in strips of rows and shuffled:
+//   all workgroups on the chip at once        1.04-2.3 (shuffled with Green-Gauss 0.95-2.1)
+//   up to two ring gradients a cell, and
+//     ten waves or more a compute unit        1.04-1.5
+//     eight, the chip filled up to 2.5 times  0.97-1.17, and beyond 0.84-1.11
+//     fewer (by rows, 64 or 128 a tile)       0.74-1.16
+//   3.5 ring gradients a cell (shuffled)      0.41-1.03
+bool one_launch_pays(long cells, long tiles, long first_ring, size_t lds, int block) {
+    constexpr size_t kWorkgroupLds = 65536, kUnitLds = 163840;
+    constexpr long kUnits = 256;
+    if (lds > kWorkgroupLds) return false;
+    const long per_unit = (long)(kUnitLds / lds);
+    if (tiles <= per_unit * kUnits) return true;
+    const long waves = per_unit * block / 64;
+    return first_ring <= 2 * cells && (waves >= 10 || (waves >= 8 && 2 * tiles <= 5 * per_unit * kUnits));
 }
 
 // Calls f(cell, slot, face entry, cell is the entry's right cell) for every used face slot.

@@ -1,6 +1,7 @@
 // Host-side mesh processing: the reference's connectivity and geometry, and the tiled,
 // renumbered layout the kernels use.
 #pragma once
+#include <cstddef>
 #include <cstdint>
 #include <vector>
 
@@ -62,6 +63,7 @@ struct TileRings {
     bool ok = false;             // false: a tile has more local cells than 16-bit indices hold
     int max_local = 0;           // most local cells of a tile
     int max_grad = 0;            // most own and first-ring cells of a tile (those with gradients)
+    long first_ring = 0;         // first-ring cells of all tiles
     std::vector<int> tiles;      // [4*ntiles] {ring start, n1 | ghosts << 16, nr, ghost start}
     std::vector<int> cell;       // ring cells of the tiles in turn (renumbered), first then second ring
     std::vector<uint16_t> own;   // [4*nc] local neighbours of each cell in its own tile, face order; 0xFFFF = none
@@ -71,6 +73,9 @@ struct TileRings {
     std::vector<uint16_t> face;  // [2*face entries] local cells of L and R (R: the ghost on a boundary face)
 };
 void tile_rings(const RefMesh &m, const Layout &L, TileRings &r);
+// Whether a pass that forms its tiles' gradients itself is the faster form, for workgroups of `block`
+// threads and `lds` bytes.
+bool one_launch_pays(long cells, long tiles, long first_ring, std::size_t lds, int block);
 
 // Per cell and face slot, renumbered cells: the least-squares vector (w, 8 doubles per cell), and
 // the outward unit normal and length (n, 12 doubles per cell); zero for unused slots.
