@@ -19,6 +19,11 @@
 // every variant that spilled (a second prefetched stencil for Green-Gauss, initialised records) lost
 // more than it hid.
 //
+// The recomputing pass forms a marked tile's gradients again, where the two-pass form reads them. With few
+// marked tiles that is free; with nearly all of them marked (a 2.6M-cell bump with 30 % noise in every cell,
+// RK4 steps in tiles of 128) the two-pass form takes 3.36 ms with HLLC and 3.56 with Roe and Green-Gauss,
+// this one 3.50 and 3.91 (3.61 and 4.10 with a flux evaluation for each kind of face).
+//
 // Local cells of a tile: its own cells, the first ring (whose gradients the tile's faces read), the
 // second ring (whose states the first ring's gradients read) and the ghosts of boundary faces
 // (mesh_host.h, TileRings). Phases:
@@ -137,22 +142,23 @@ __device__ __forceinline__ void fused_face(const FusedArgs &A, const double2 *sW
     const bool boundary = lc.y >= t.nct + t.nr;
     int kind = 0;
     if (boundary) kind = A.m.ghost[t.g0 + lc.y - t.nct - t.nr].y;
+    FState SL, SR, fL, fR;
+    double gL[8], gR[8];
+    bool first = false;
     if constexpr (POS == 2) {
         // positivity fallback, recomputation: a face of a flagged cell takes the two cells'
-        // first-order states (conserved values as stored, ghost of the left state)
+        // first-order states (conserved values as stored, ghost of the left state). Both kinds of face
+        // share the flux below, which a wave of both would otherwise go through twice
         const uint8_t *pflag = A.st.pflag;
         const int L = local_cell(A.m, lc.x, t.c0, t.nct, t.r0);
         const int R = boundary ? L : local_cell(A.m, lc.y, t.c0, t.nct, t.r0);
-        if (pflag[L] || pflag[R]) {
-            FState SL, SR;
-            load_state(A.Us, L, SL);
-            if (boundary) ghost_of_tile(A, t.tile, kind, SL, nx, ny, SR);
-            else load_state(A.Us, R, SR);
-            face_flux<FLUX>(boundary, A.cfg.roe_bdiss, SL, SR, nx, ny, dl, F);
-            return;
+        first = pflag[L] || pflag[R];
+        if (first) {
+            load_state(A.Us, L, fL);
+            if (boundary) ghost_of_tile(A, t.tile, kind, fL, nx, ny, fR);
+            else load_state(A.Us, R, fR);
         }
     }
-    FState SL, SR, fL, fR;
     auto prims = [&](int l, FState &s) {
         const double2 a = sWa[l], b = sWb[l];
         s.W[0] = a.x;
@@ -167,30 +173,31 @@ __device__ __forceinline__ void fused_face(const FusedArgs &A, const double2 *sW
             g[2 * q + 1] = v.y;
         }
     };
-    prims(lc.x, SL);
-    prims(lc.y, SR);
-    double gL[8], gR[8];
-    // frozen limiter factors of this face entry (8 floats, two 16-byte loads)
-    float pv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float4 *p4 = fz ? reinterpret_cast<float4 *>(A.st.psi) + 2 * (size_t)e : nullptr;
-    if (fz == 2) {
-        const float4 a = p4[0], b = p4[1];
-        pv[0] = a.x; pv[1] = a.y; pv[2] = a.z; pv[3] = a.w;
-        pv[4] = b.x; pv[5] = b.y; pv[6] = b.z; pv[7] = b.w;
-    }
-    gradient(lc.x, gL);
-    reconstruct_side<LIM, false>(SL, SR, gL, f.dx, f.dy, 1.0, fz, pv, fL);
-    if (boundary) {
-        ghost_of_tile(A, t.tile, kind, fL, nx, ny, fR);
-        if constexpr (VISC)
-            for (int q = 0; q < 8; q++) gR[q] = gL[q];
-    } else {
-        gradient(lc.y, gR);
-        reconstruct_side<LIM, false>(SR, SL, gR, f.dx, f.dy, -1.0, fz, pv + 4, fR);
-    }
-    if (fz == 1) {
-        p4[0] = make_float4(pv[0], pv[1], pv[2], pv[3]);
-        p4[1] = make_float4(pv[4], pv[5], pv[6], pv[7]);
+    if (!first) {
+        prims(lc.x, SL);
+        prims(lc.y, SR);
+        // frozen limiter factors of this face entry (8 floats, two 16-byte loads)
+        float pv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        float4 *p4 = fz ? reinterpret_cast<float4 *>(A.st.psi) + 2 * (size_t)e : nullptr;
+        if (fz == 2) {
+            const float4 a = p4[0], b = p4[1];
+            pv[0] = a.x; pv[1] = a.y; pv[2] = a.z; pv[3] = a.w;
+            pv[4] = b.x; pv[5] = b.y; pv[6] = b.z; pv[7] = b.w;
+        }
+        gradient(lc.x, gL);
+        reconstruct_side<LIM, false>(SL, SR, gL, f.dx, f.dy, 1.0, fz, pv, fL);
+        if (boundary) {
+            ghost_of_tile(A, t.tile, kind, fL, nx, ny, fR);
+            if constexpr (VISC)
+                for (int q = 0; q < 8; q++) gR[q] = gL[q];
+        } else {
+            gradient(lc.y, gR);
+            reconstruct_side<LIM, false>(SR, SL, gR, f.dx, f.dy, -1.0, fz, pv + 4, fR);
+        }
+        if (fz == 1) {
+            p4[0] = make_float4(pv[0], pv[1], pv[2], pv[3]);
+            p4[1] = make_float4(pv[4], pv[5], pv[6], pv[7]);
+        }
     }
     face_flux<FLUX>(boundary, A.cfg.roe_bdiss, fL, fR, nx, ny, dl, F);
     if constexpr (VISC) {
