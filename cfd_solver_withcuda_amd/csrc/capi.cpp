@@ -5,11 +5,13 @@
 
 #include <cmath>
 #include <cstring>
+#include <future>
 #include <memory>
 #include <mutex>
 #include <new>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <vector>
 
 #include "capi_internal.h"
@@ -45,6 +47,43 @@ hipError_t upload(T **d, const std::vector<T> &h) {
     if (e != hipSuccess) return e;
     return hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice);
 }
+
+// Host arrays copied into one device allocation. An allocation and a copy for each of a mesh's two dozen
+// arrays were the larger part of creating a small one: 385 -> 73 us for 43 cells.
+class DeviceBlock {
+    struct Part {
+        void **d;
+        const void *h;
+        size_t bytes, at;
+    };
+    std::vector<Part> parts_;
+    size_t total_ = 0;
+
+  public:
+    // *d points to the copy of h (null if h is empty) once uploaded; h stays until then.
+    template <typename T>
+    void add(T **d, const std::vector<T> &h) {
+        *d = nullptr;
+        if (h.empty()) return;
+        parts_.push_back({(void **)d, h.data(), h.size() * sizeof(T), total_});
+        total_ = (total_ + h.size() * sizeof(T) + 255) / 256 * 256;
+    }
+    hipError_t upload(void **block) {
+        if (!total_) return hipSuccess;
+        hipError_t e = hipMalloc(block, total_);
+        if (e != hipSuccess) return e;
+        char *base = (char *)*block;
+        for (const Part &p : parts_) *p.d = base + p.at;
+        if (total_ <= (size_t)1 << 20) {  // one copy
+            std::vector<char> all(total_);
+            for (const Part &p : parts_) std::memcpy(&all[p.at], p.h, p.bytes);
+            return hipMemcpy(base, all.data(), total_, hipMemcpyHostToDevice);
+        }
+        for (const Part &p : parts_)
+            if ((e = hipMemcpy(base + p.at, p.h, p.bytes, hipMemcpyHostToDevice)) != hipSuccess) return e;
+        return hipSuccess;
+    }
+};
 
 }  // namespace
 
@@ -220,6 +259,62 @@ int cfd_mesh_create_host(int npts, const double *pts3, int ncells, const int *ce
     return 0;
 }
 
+// The device arrays of a mesh. The tiles' neighbourhoods are built beside the packing and the copies of
+// the rest, which take longer; every mesh has them, since cfd_residual_noalloc may not allocate them later.
+static hipError_t upload_mesh(cfd_mesh_s *m, TileRings &rings) {
+    const Layout &L = m->lay;
+    std::future<void> built;
+    auto build = [&]() { tile_rings(m->ref, L, rings); };
+    try {
+        if (m->ref.nc >= 2048) built = std::async(std::launch::async, build);
+    } catch (const std::system_error &) {  // no thread to be had: built below
+    }
+    std::vector<double> geo, cw, fd;
+    std::vector<int> lr;
+    pack_face_geometry(L, 0, geo, lr);
+    cell_face_vectors(L, cw);
+    face_offsets(L, fd);
+    const RefMesh &R = m->ref;
+    std::vector<int> gc(R.ng), gk(R.ng);
+    std::vector<double> gn(2 * (size_t)R.ng);
+    for (int k = 0; k < R.ng; k++) {
+        const int c = R.gcell[k], f = R.gface[k];
+        gc[k] = L.iperm[c];
+        gk[k] = R.kind[4 * c + f];
+        gn[2 * k] = R.nrm[8 * c + 2 * f];
+        gn[2 * k + 1] = R.nrm[8 * c + 2 * f + 1];
+    }
+    DeviceBlock base;
+    base.add(&m->d_tile_cstart, L.tile_cstart);
+    base.add(&m->d_tile_fstart, L.tile_fstart);
+    base.add(&m->d_fgeo, geo);
+    base.add(&m->d_cw, cw);
+    base.add(&m->d_fd, fd);
+    base.add(&m->d_fLR, lr);
+    base.add(&m->d_fnx, L.fnx);
+    base.add(&m->d_fny, L.fny);
+    base.add(&m->d_fdl, L.fdl);
+    base.add(&m->d_slots, L.slots);
+    base.add(&m->d_area, L.area);
+    base.add(&m->d_inv_area, L.inv_area);
+    base.add(&m->d_gcell, gc);
+    base.add(&m->d_gkind, gk);
+    base.add(&m->d_gnrm, gn);
+    const hipError_t e = base.upload(&m->d_base);
+    if (built.valid()) built.get();
+    else build();
+    if (e != hipSuccess || !rings.ok) return e;
+    DeviceBlock nb;
+    nb.add(&m->d_rings, rings.tiles);
+    nb.add(&m->d_ring_cell, rings.cell);
+    nb.add(&m->d_own_nbr, rings.own);
+    nb.add(&m->d_ring_nbr, rings.ring);
+    nb.add(&m->d_ghost, rings.ghost);
+    nb.add(&m->d_ghost_n, rings.ghost_n);
+    nb.add(&m->d_floc, rings.face);
+    return nb.upload(&m->d_neighbourhoods);
+}
+
 int cfd_mesh_create(int npts, const double *pts3, int ncells, const int *cells4, int tile,
                     int face_budget, int renumber, cfd_mesh_t **out) {
     int rc = cfd_mesh_create_host(npts, pts3, ncells, cells4, tile, face_budget, renumber, out);
@@ -227,45 +322,16 @@ int cfd_mesh_create(int npts, const double *pts3, int ncells, const int *cells4,
     cfd_mesh_s *m = *out;
     *out = nullptr;
     const Layout &L = m->lay;
-    hipError_t e = hipSuccess;
-    std::vector<double> geo, cw, fd;
-    std::vector<int> lr;
-    pack_face_geometry(L, 0, geo, lr);
-    cell_face_vectors(L, cw);
-    face_offsets(L, fd);
     TileRings rings;
-    tile_rings(m->ref, L, rings);
-    if ((e = upload(&m->d_tile_cstart, L.tile_cstart)) != hipSuccess ||
-        (e = upload(&m->d_tile_fstart, L.tile_fstart)) != hipSuccess ||
-        (e = upload(&m->d_fgeo, geo)) != hipSuccess || (e = upload(&m->d_cw, cw)) != hipSuccess ||
-        (e = upload(&m->d_fd, fd)) != hipSuccess ||
-        (e = upload(&m->d_rings, rings.tiles)) != hipSuccess || (e = upload(&m->d_ring_cell, rings.cell)) != hipSuccess ||
-        (e = upload(&m->d_own_nbr, rings.own)) != hipSuccess || (e = upload(&m->d_ring_nbr, rings.ring)) != hipSuccess ||
-        (e = upload(&m->d_ghost, rings.ghost)) != hipSuccess ||
-        (e = upload(&m->d_ghost_n, rings.ghost_n)) != hipSuccess || (e = upload(&m->d_floc, rings.face)) != hipSuccess ||
-        (e = upload(&m->d_fLR, lr)) != hipSuccess || (e = upload(&m->d_fnx, L.fnx)) != hipSuccess ||
-        (e = upload(&m->d_fny, L.fny)) != hipSuccess || (e = upload(&m->d_fdl, L.fdl)) != hipSuccess ||
-        (e = upload(&m->d_slots, L.slots)) != hipSuccess ||
-        (e = upload(&m->d_area, L.area)) != hipSuccess || (e = upload(&m->d_inv_area, L.inv_area)) != hipSuccess) {
-        delete m;
-        return hip_fail(e, "cfd_mesh_create upload");
-    }
-    {
-        const RefMesh &R = m->ref;
-        std::vector<int> gc(R.ng), gk(R.ng);
-        std::vector<double> gn(2 * (size_t)R.ng);
-        for (int k = 0; k < R.ng; k++) {
-            const int c = R.gcell[k], f = R.gface[k];
-            gc[k] = L.iperm[c];
-            gk[k] = R.kind[4 * c + f];
-            gn[2 * k] = R.nrm[8 * c + 2 * f];
-            gn[2 * k + 1] = R.nrm[8 * c + 2 * f + 1];
-        }
-        if ((e = upload(&m->d_gcell, gc)) != hipSuccess || (e = upload(&m->d_gkind, gk)) != hipSuccess ||
-            (e = upload(&m->d_gnrm, gn)) != hipSuccess) {
+    try {
+        const hipError_t e = upload_mesh(m, rings);
+        if (e != hipSuccess) {
             delete m;
             return hip_fail(e, "cfd_mesh_create upload");
         }
+    } catch (const std::exception &e) {  // out of host memory
+        delete m;
+        return fail(CFD_E_MESH, std::string("cfd_mesh_create: ") + e.what());
     }
     DevMesh &d = m->dev;
     d.nc = m->ref.nc;
@@ -429,7 +495,11 @@ static int ensure_cell_normals(cfd_mesh_s *m) {
     std::lock_guard<std::mutex> lock(m->lazy);
     if (m->d_cn || !m->dev.rings) return 0;
     std::vector<double> cn;
-    cell_face_normals(m->lay, cn);
+    try {
+        cell_face_normals(m->lay, cn);
+    } catch (const std::exception &e) {
+        return fail(CFD_E_MESH, std::string("cell normals: ") + e.what());
+    }
     HIP_TRY(upload(&m->d_cn, cn));
     m->dev.cn = m->d_cn;
     return 0;

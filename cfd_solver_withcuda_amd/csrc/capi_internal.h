@@ -18,16 +18,19 @@ struct cfd_mesh_s {
     RefMesh ref;
     Layout lay;
     bool on_device = false;
+    void *d_base = nullptr, *d_neighbourhoods = nullptr;  // hold the arrays of the next two groups
     int *d_tile_cstart = nullptr, *d_tile_fstart = nullptr;
-    double *d_fgeo = nullptr, *d_cw = nullptr, *d_cn = nullptr, *d_ghost_n = nullptr, *d_fd = nullptr, *d_fnx = nullptr, *d_fny = nullptr, *d_fdl = nullptr;
+    double *d_fgeo = nullptr, *d_cw = nullptr, *d_fd = nullptr, *d_fnx = nullptr, *d_fny = nullptr, *d_fdl = nullptr;
     int *d_fLR = nullptr;
     uint16_t *d_slots = nullptr;
-    // tile neighbourhoods (TileRings)
-    int *d_rings = nullptr, *d_ring_cell = nullptr, *d_ghost = nullptr;
-    uint16_t *d_own_nbr = nullptr, *d_ring_nbr = nullptr, *d_floc = nullptr;
     double *d_area = nullptr, *d_inv_area = nullptr;
     int *d_gcell = nullptr, *d_gkind = nullptr;  // ghost k: renumbered owner cell, face kind
     double *d_gnrm = nullptr;                    // ghost k: unit normal of the owner's face
+    // tile neighbourhoods (TileRings)
+    int *d_rings = nullptr, *d_ring_cell = nullptr, *d_ghost = nullptr;
+    double *d_ghost_n = nullptr;
+    uint16_t *d_own_nbr = nullptr, *d_ring_nbr = nullptr, *d_floc = nullptr;
+    double *d_cn = nullptr;  // face normals per cell (built on first use by Green-Gauss)
     // the reference's per-cell arrays in renumbered order (built on first use by the reference's
     // second order)
     int *d_rc_nf = nullptr, *d_rc_nbr = nullptr;
@@ -40,9 +43,7 @@ struct cfd_mesh_s {
     mutable std::mutex lazy;  // guards the arrays built on first use (solvers may share the mesh)
     DevMesh dev{};
     ~cfd_mesh_s() {
-        void *ps[] = {d_tile_cstart, d_tile_fstart, d_fgeo, d_cw, d_cn, d_ghost_n, d_fd, d_fnx, d_fny, d_fdl, d_fLR, d_slots, d_rings, d_ring_cell, d_ghost, d_own_nbr,
-                      d_ring_nbr, d_floc, d_area, d_inv_area, d_gcell, d_gkind, d_gnrm,
-                      d_rc_nf, d_rc_nbr, d_rc_dist, d_rc_nrm, d_rc_len, d_rc_area, d_fst, d_gtiles, d_gcount};
+        void *ps[] = {d_base, d_neighbourhoods, d_cn, d_rc_nf, d_rc_nbr, d_rc_dist, d_rc_nrm, d_rc_len, d_rc_area, d_fst, d_gtiles, d_gcount};
         for (void *p : ps)
             if (p) (void)hipFree(p);
     }
