@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "fv_kernels.h"
+#include "host_ahead.h"
 #include "host_rows.h"
 #include "mesh_host.h"
 
@@ -170,14 +171,7 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
     std::vector<Layout> lays(ni);
     std::vector<std::vector<int>> sts(ni);  // WENO line stencils (order 3)
     std::vector<TileRings> rgs(ni);         // tile neighbourhoods (order 2)
-    struct Packed {                         // the instance's device records
-        std::vector<double> geo, cw, cn, fd;
-        std::vector<int> lr;
-    };
-    std::vector<Packed> pks(ni);
     std::vector<std::string> errs(ni);
-    std::vector<long> first_cell(ni + 1, 0);
-    for (int i = 0; i < ni; i++) first_cell[i + 1] = first_cell[i] + in[i].ncells;
     {
         std::atomic<int> next{0};
         auto work = [&]() {
@@ -189,14 +183,7 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
                     build_ref_mesh(in[i].npts, in[i].pts, in[i].ncells, in[i].cells, rm);
                     build_layout(rm, tile, 1, lays[i], face_budget);
                     if (cfg.order == 3) line_stencils(rm, lays[i], sts[i]);
-                    Packed &pk = pks[i];
-                    pack_face_geometry(lays[i], (int)first_cell[i], pk.geo, pk.lr);
-                    if (cfg.order >= 2) cell_face_vectors(lays[i], pk.cw);
-                    if (cfg.order == 2) {
-                        tile_rings(rm, lays[i], rgs[i]);
-                        face_offsets(lays[i], pk.fd);
-                        if (cfg.gradient == GRAD_GG) cell_face_normals(lays[i], pk.cn);
-                    }
+                    if (cfg.order == 2) tile_rings(rm, lays[i], rgs[i]);
                 } catch (const std::exception &e) {
                     errs[i] = e.what();
                 }
@@ -304,66 +291,118 @@ int build_batch(const std::vector<InstanceInput> &in, const double *fs4, const c
     }
 #undef BALLOC
     b->iperm.resize(nc);
-    for (int i = 0; i < ni; i++) {
-        Layout &L = lays[i];
-        const int cb = b->cell_off[i], tb = b->inst_tile[i], fb = fe_off[i];
-        const size_t nci = L.area.size(), nti = L.ntiles, nfi = L.fL.size();
-        std::vector<int> tc(nti), tf(nti), ti(nti, i);
-        for (size_t t = 0; t < nti; t++) {
-            tc[t] = L.tile_cstart[t] + cb;
-            tf[t] = L.tile_fstart[t] + fb;
-        }
-        Packed &pk = pks[i];
-        if (rings) {
-            TileRings &rg = rgs[i];
-            for (size_t t = 0; t < nti; t++) {
-                rg.tiles[4 * t] += (int)rc_off[i];
-                rg.tiles[4 * t + 3] += (int)gh_off[i];
+    // The device records, 200 to 300 bytes a cell beside the layouts: packed by other threads, a few groups
+    // of instances ahead, while the groups before are copied. A group is an instance, or several small ones
+    // in a row, whose arrays go in one copy each (creating 256 instances of 2k cells: 95 ms with copies of
+    // every instance's, 36 so).
+    constexpr size_t kGroupCells = 32768;
+    std::vector<int> group(1, 0);  // first instance of each group, and the end
+    for (int i = 1; i <= ni; i++)
+        if (i == ni || (size_t)(b->cell_off[i + 1] - b->cell_off[group.back()]) > kGroupCells) group.push_back(i);
+    struct Packed {
+        std::vector<double> geo, cw, cn, fd, fnx, fny, fdl, area, inv_area, ghost_n;
+        std::vector<int> lr, tc, tf, ti, st, rings, ring_cell, ghost;
+        std::vector<uint16_t> slots, own, ring, face;
+    };
+    auto pack = [&](int g) {
+        Packed pk;
+        auto add = [](auto &all, auto &&part) {
+            if (all.empty()) all = std::move(part);
+            else all.insert(all.end(), part.begin(), part.end());
+        };
+        for (int i = group[g]; i < group[g + 1]; i++) {
+            Layout L = std::move(lays[i]);
+            TileRings rg = std::move(rgs[i]);
+            std::vector<int> st = std::move(sts[i]);
+            const int cb = b->cell_off[i], fb = fe_off[i];
+            std::vector<double> geo, v;
+            std::vector<int> lr;
+            pack_face_geometry(L, cb, geo, lr);
+            add(pk.geo, std::move(geo));
+            add(pk.lr, std::move(lr));
+            if (cfg.order >= 2) {
+                cell_face_vectors(L, v);
+                add(pk.cw, std::move(v));
             }
-            for (int &v : rg.cell) v += cb;
-            for (size_t g = 0; g < rg.ghost.size(); g += 2) rg.ghost[g] += cb;
-            if ((e = h2d(b->d_rings + 4 * (size_t)tb, rg.tiles.data(), rg.tiles.size())) != hipSuccess ||
-                (e = h2d(b->d_ring_cell + rc_off[i], rg.cell.data(), rg.cell.size())) != hipSuccess ||
-                (e = h2d(b->d_own_nbr + 4 * (size_t)cb, rg.own.data(), rg.own.size())) != hipSuccess ||
-                (e = h2d(b->d_ring_nbr + 4 * rc_off[i], rg.ring.data(), rg.ring.size())) != hipSuccess ||
-                (e = h2d(b->d_ghost + 2 * gh_off[i], rg.ghost.data(), rg.ghost.size())) != hipSuccess ||
-                (e = h2d(b->d_ghost_n + 2 * gh_off[i], rg.ghost_n.data(), rg.ghost_n.size())) != hipSuccess ||
-                (e = h2d(b->d_floc + 2 * (size_t)fb, rg.face.data(), rg.face.size())) != hipSuccess ||
-                (e = h2d(b->d_fd + 2 * (size_t)fb, pk.fd.data(), pk.fd.size())) != hipSuccess ||
-                (b->d_cn && (e = h2d(b->d_cn + 12 * (size_t)cb, pk.cn.data(), pk.cn.size())) != hipSuccess)) {
-                delete b;
-                return capi_hip_fail(e, "cfd_batch_create upload");
+            if (rings) {
+                face_offsets(L, v);
+                add(pk.fd, std::move(v));
+                if (cfg.gradient == GRAD_GG) {
+                    cell_face_normals(L, v);
+                    add(pk.cn, std::move(v));
+                }
+                for (size_t t = 0; t < (size_t)L.ntiles; t++) {
+                    rg.tiles[4 * t] += (int)rc_off[i];
+                    rg.tiles[4 * t + 3] += (int)gh_off[i];
+                }
+                for (int &c : rg.cell) c += cb;
+                for (size_t k = 0; k < rg.ghost.size(); k += 2) rg.ghost[k] += cb;
+                add(pk.rings, std::move(rg.tiles));
+                add(pk.ring_cell, std::move(rg.cell));
+                add(pk.own, std::move(rg.own));
+                add(pk.ring, std::move(rg.ring));
+                add(pk.ghost, std::move(rg.ghost));
+                add(pk.ghost_n, std::move(rg.ghost_n));
+                add(pk.face, std::move(rg.face));
             }
-            rg = TileRings();
-        }
-        if (cfg.order == 3) {
-            std::vector<int> &st = sts[i];
-            for (int &v : st)
-                if (v >= 0) v += cb;
-            if ((e = h2d(b->d_fst + 4 * (size_t)fb, st.data(), 4 * nfi)) != hipSuccess) {
-                delete b;
-                return capi_hip_fail(e, "cfd_batch_create upload");
+            for (int &c : st)
+                if (c >= 0) c += cb;
+            add(pk.st, std::move(st));
+            pk.ti.insert(pk.ti.end(), L.ntiles, i);
+            for (int t = 0; t < L.ntiles; t++) {
+                pk.tc.push_back(L.tile_cstart[t] + cb);
+                pk.tf.push_back(L.tile_fstart[t] + fb);
             }
-            std::vector<int>().swap(st);
+            for (size_t c = 0; c < L.iperm.size(); c++) b->iperm[cb + c] = cb + L.iperm[c];
+            add(pk.fnx, std::move(L.fnx));
+            add(pk.fny, std::move(L.fny));
+            add(pk.fdl, std::move(L.fdl));
+            add(pk.slots, std::move(L.slots));
+            add(pk.area, std::move(L.area));
+            add(pk.inv_area, std::move(L.inv_area));
         }
-        for (size_t c = 0; c < nci; c++) b->iperm[cb + c] = cb + L.iperm[c];
-        if ((e = h2d(b->d_tile_cstart + tb, tc.data(), nti)) != hipSuccess ||
-            (e = h2d(b->d_tile_fstart + tb, tf.data(), nti)) != hipSuccess ||
-            (e = h2d(b->d_tile_inst + tb, ti.data(), nti)) != hipSuccess ||
-            (e = h2d(b->d_fgeo + 6 * (size_t)fb, pk.geo.data(), 6 * nfi)) != hipSuccess ||
-            (b->d_cw && (e = h2d(b->d_cw + 8 * (size_t)cb, pk.cw.data(), pk.cw.size())) != hipSuccess) ||
-            (e = h2d(b->d_fLR + 2 * (size_t)fb, pk.lr.data(), 2 * nfi)) != hipSuccess ||
-            (e = h2d(b->d_fnx + fb, L.fnx.data(), nfi)) != hipSuccess ||
-            (e = h2d(b->d_fny + fb, L.fny.data(), nfi)) != hipSuccess ||
-            (e = h2d(b->d_fdl + fb, L.fdl.data(), nfi)) != hipSuccess ||
-            (e = h2d(b->d_slots + 4 * (size_t)cb, L.slots.data(), 4 * nci)) != hipSuccess ||
-            (e = h2d(b->d_area + cb, L.area.data(), nci)) != hipSuccess ||
-            (e = h2d(b->d_inv_area + cb, L.inv_area.data(), nci)) != hipSuccess) {
-            delete b;
-            return capi_hip_fail(e, "cfd_batch_create upload");
-        }
-        L = Layout();  // release this instance's host copies
-        pk = Packed();
+        return pk;
+    };
+    auto copy = [&](int g, const Packed &pk) {
+        const int i = group[g];
+        const size_t cb = b->cell_off[i], tb = b->inst_tile[i], fb = fe_off[i];
+        auto put = [&](auto *d, size_t at, const auto &v) {
+            if (e == hipSuccess && d) e = h2d(d + at, v.data(), v.size());
+        };
+        put(b->d_tile_cstart, tb, pk.tc);
+        put(b->d_tile_fstart, tb, pk.tf);
+        put(b->d_tile_inst, tb, pk.ti);
+        put(b->d_fgeo, 6 * fb, pk.geo);
+        put(b->d_cw, 8 * cb, pk.cw);
+        put(b->d_fLR, 2 * fb, pk.lr);
+        put(b->d_fst, 4 * fb, pk.st);
+        put(b->d_fnx, fb, pk.fnx);
+        put(b->d_fny, fb, pk.fny);
+        put(b->d_fdl, fb, pk.fdl);
+        put(b->d_slots, 4 * cb, pk.slots);
+        put(b->d_area, cb, pk.area);
+        put(b->d_inv_area, cb, pk.inv_area);
+        put(b->d_rings, 4 * tb, pk.rings);
+        put(b->d_ring_cell, rc_off[i], pk.ring_cell);
+        put(b->d_own_nbr, 4 * cb, pk.own);
+        put(b->d_ring_nbr, 4 * rc_off[i], pk.ring);
+        put(b->d_ghost, 2 * gh_off[i], pk.ghost);
+        put(b->d_ghost_n, 2 * gh_off[i], pk.ghost_n);
+        put(b->d_floc, 2 * fb, pk.face);
+        put(b->d_fd, 2 * fb, pk.fd);
+        put(b->d_cn, 12 * cb, pk.cn);
+        return e == hipSuccess;
+    };
+    try {
+        const int groups = (int)group.size() - 1;
+        in_turn(groups, std::max(1, std::min(nthreads, groups)) - 1, pack, copy);
+    } catch (const std::exception &x) {
+        delete b;
+        return capi_fail(CFD_E_MESH, std::string("cfd_batch_create: ") + x.what());
+    }
+    if (e != hipSuccess) {
+        delete b;
+        return capi_hip_fail(e, "cfd_batch_create upload");
     }
     const int last_c = b->nc, last_f = b->nfe;
     std::vector<double4> fsv(ni);
