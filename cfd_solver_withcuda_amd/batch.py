@@ -3,7 +3,7 @@
 Many independent meshes of uneven size (the reference solves one Inviscid_Solver case per run,
 src/Solver.cpp:93-118) are concatenated into one device mesh and marched together with local
 time stepping until each instance's Error[0] (Estimate_Error, src/Error_Estimate_Update.cpp:10-30)
-reaches the tolerance. One RK step of all instances is one hipGraph launch; converged instances
+reaches the tolerance. Steps of all instances are captured in hipGraphs (one or eight to a graph); converged instances
 drop out of the tile list on the device.
 """
 from __future__ import annotations

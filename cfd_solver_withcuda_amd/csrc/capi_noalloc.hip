@@ -1,8 +1,8 @@
 // Allocation-free residual entry point (cfd_residual_noalloc, include/cfd_hip.h).
 //
-// It runs the kernels of cfd_residual (gradient pass, flux pass in residual mode, minimum of the
-// local time steps) on a caller's device state. The gradients and the per-tile time-step minima
-// those kernels need live in `scratch`, a file-scope device array of fixed size, so the call
+// It runs the kernels of cfd_residual (the second-order residual in one launch, or gradients and then
+// fluxes; minimum of the local time steps) on a caller's device state. The gradients of the two launches
+// and the per-tile time-step minima live in `scratch`, a file-scope device array of fixed size, so the call
 // allocates nothing: no hipMalloc, no hipFree, no allocating library routine. Each device that
 // loads the library holds its own copy of the array until the process ends; its address on a
 // device is looked up once, with that device current, on the first call there.

@@ -568,8 +568,9 @@ __device__ __forceinline__ double plain_div(double a, double b, double y) {
 }
 
 // The two face values of weno5 (a, b, c | d, e, f: left with shift 0, right with shift 1) for inputs
-// below 2^200, where every square and quotient of the weights is normal. A NaN among a value's inputs makes
-// it one.
+// below 2^200, where every square and quotient of the weights is normal. The stencils' values, quotients by
+// 6, are subnormal only with every input below 1e-290; their last bit, 5e-324, can then be another than the
+// division's. A NaN among a value's inputs makes it one.
 __device__ __forceinline__ void weno5_pair(double a, double b, double c, double d, double e, double f, double &UL,
                                            double &UR) {
     const double eps = 1e-6, y6 = 1.0 / 6.0;

@@ -14,7 +14,7 @@
 // in registers to 2.61 ms, 0.307 ms, 113 us and 31 us).
 //
 // What bounds it (forward step, 0.65 ms a stage): FP64 issue, about 2,000 vector instructions a wave or
-// 70-75 % of the launch; the L2 fills run at 4.4-4.9 TB/s, the rate of a large copy on the same card.
+// 70-75 % of the launch; the L2 fills run at 4.4-4.9 TB/s, the rate (4.7) of a copy of arrays beyond the last-level cache.
 // Neither leaves room for less occupancy: 128 registers and 20 KB of LDS give 4 waves per SIMD, and
 // every variant that spilled (a second prefetched stencil for Green-Gauss, initialised records) lost
 // more than it hid.

@@ -1,5 +1,5 @@
 // Training step and prediction of the surrogate MLP for networks of up to 256 (padded) features a
-// layer, in three launches a step:
+// layer (and 32 outputs, the most that a network may have), in three launches a step:
 //   rows    a workgroup takes 32 samples through the whole network and, in training, back again:
 //           activations and gradients stay in LDS from layer to layer, weights stream from L2 (one
 //           layer ahead, in registers, laid out as the matrix instructions take them). Layer by layer
@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(256) wgrad_kernel(MlpLayers T, int rows, int s
 // ---- sums of the row ranges, then Adam -------------------------------------------------------
 // A workgroup takes a 32 x 32 tile of a layer's weights (four in a row per thread), or eight
 // biases, whose gradients it sums over the rows (row_sum_layers_kernel's parts and order). Bound by the
-// reads of P and dZt, 42 MB each at 16384 rows of 6 x 256: 20 us, with one bias a workgroup 26 us.
+// reads of P and dZt, 44 and 52 MB at 16384 rows of 6 x 256: 20 us, with one bias a workgroup 26 us.
 template <bool ADAM>
 __global__ void __launch_bounds__(256) update_kernel(MlpLayers T, const float *P, int split, int rows, int biases, MlpAdam a,
                                                      float *gW, float *gb) {

@@ -239,8 +239,9 @@ class Solver:
         return None
 
     def time_pass(self, which: str, reps: int, stream: int = 0) -> float:
-        """Milliseconds for `reps` launches of 'grad', 'flux' (fused stage), 'step' or 'resid' (the
-        flux pass in residual mode) (HIP events)."""
+        """Milliseconds (HIP events) for `reps` launches of 'flux' (a step's first stage), 'resid' (the
+        residual), 'step' (whole steps) or 'grad' (the gradient kernel). A second-order stage or residual
+        that is one launch forms its gradients itself: 'grad' is no part of it."""
         ms = ctypes.c_float()
         check(lib().cfd_time_pass(self.h, dict(grad=0, flux=1, step=2, resid=3)[which], reps,
                                   ctypes.byref(ms), ctypes.c_void_p(stream)), "cfd_time_pass")

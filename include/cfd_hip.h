@@ -178,11 +178,15 @@ int cfd_step(cfd_solver_t *s, int nsteps, double *err_hist, double *dt_hist, voi
 int cfd_run_steady(cfd_solver_t *s, double tol, int max_steps, int check_every, int *steps,
                    double *err4, void *stream);
 
-/* Times `reps` back-to-back launches on `stream` with HIP events: which = 0 the gradient pass,
- * 1 the fused flux/stage pass (first stage, output to scratch; the state is unchanged; with the
- * positivity fallback its detecting pass),
- * 2 whole steps (advances the state), 3 the flux pass in residual mode (R and the local time
- * step out, as cfd_residual). *ms = total elapsed milliseconds. */
+/* Times `reps` back-to-back launches on `stream` with HIP events. *ms = total elapsed milliseconds.
+ *   which = 0  the gradient kernel. At order 2 a step or residual launches it only where it takes two
+ *              launches (cells in the caller's own order that scatter the tiles, the reference
+ *              iteration); otherwise 1 and 3 form the gradients themselves, and 0 is no part of them
+ *           1  a step's first stage (output to scratch; the state is unchanged; with the positivity
+ *              fallback its detecting pass). Order 2: gradients included where it is one launch; orders
+ *              1 and 3, and two-launch order 2: the flux launch alone
+ *           2  whole steps (advances the state)
+ *           3  the residual (R and the local time step out, as cfd_residual), gradients as in 1 */
 int cfd_time_pass(cfd_solver_t *s, int which, int reps, float *ms, void *stream);
 
 /* ---- batched steady solves ------------------------------------------------------------------
@@ -212,7 +216,8 @@ int cfd_batch_tuning(const cfd_batch_t *b, int *source);
 /* U[4*total cells] conserved, instances concatenated in order, each in its caller's cell order */
 int cfd_batch_set_state(cfd_batch_t *b, const double *U);
 int cfd_batch_get_state(cfd_batch_t *b, double *U);
-/* March all instances (one hipGraph launch per step; the host reads the instance status every
+/* March all instances (steps captured in hipGraphs, eight to a graph in runs of 16 and more between
+ * two status checks, else one; the host reads the instance status every
  * check_every steps). Per instance: steps[ninst] taken, err4[4*ninst] last Error[0..3],
  * status[ninst] (0 converged, 1 still marching at max_steps, -1 non-finite), conv_s[ninst]
  * wall seconds at the check where it was first seen converged; *wall_s total. Any output may be
